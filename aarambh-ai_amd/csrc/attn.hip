@@ -332,7 +332,9 @@ static constexpr int AM_HD = 128;
 static constexpr int AM_WAVES = 8;          // 512 threads; wave w takes 32-token blocks w, w+8, ...
 static constexpr int AM_TAIL = AM_WAVES - 1;  // INT8 path: the wave that appends and reads the new positions
 static constexpr int AM_HAND = 2;             // old blocks the tail wave hands over beyond its tail blocks
-static constexpr int AM_SOLO = 2;             // at most this many tail blocks go to the tail wave alone
+// Rows per sequence up to which the new positions (at most two blocks) are appended inside
+// the attention kernel; prompt chunks beyond it are appended by a launch of their own.
+static constexpr int AM_DECODE_S = 32;
 static constexpr int AM_REC = AM_HD + 4;    // partial record: m, l, pad, pad, o[hd]
 static constexpr int AM_MAXCH = 32;         // chunks one merge combines
 static constexpr int AM_STAGE = 2 * 32 * AM_HD + 512;  // one INT8 block staged in LDS: K, V^T, scales
@@ -442,6 +444,75 @@ __device__ __forceinline__ void frag_out_pair(const XFrag& fo, int orow, int oco
     frag_put8_w(fo, orow, ocol, v);
 }
 
+// Cache append of a prompt chunk (S > AM_DECODE_S): workgroup = (sequence, kv head, 32-token
+// block of the cache).  The block's new rows are rounded as append_kv_token rounds them into
+// an LDS copy of the block (loaded first where the block also holds older tokens) and the
+// block goes to the cache in 16-byte runs.  One rounding per new token: appended inside the
+// attention kernel, every 16-row query tile rounded every new token again (32 / 8 heads of
+// 128, 500 rows over an empty cache: attention 296 us; now 40 us, and 10 us for this launch,
+// which is a latency chain of one row load, two wave reductions and the stores; 128 rows
+// after 384 tokens: 42 us, now 14 + 8).
+template <int KVF>
+__global__ void __launch_bounds__(256) kv_append_kernel(AttnArgs a, int nblk) {
+    constexpr int ES = KVF == KV_INT8 ? 1 : 2, KB = 32 * AM_HD * ES;  // bytes of K (and of V) per block
+    __shared__ __attribute__((aligned(16))) char st[2 * KB];
+    __shared__ __attribute__((aligned(16))) uint16_t scl[2][32];
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int bid = blockIdx.x;
+    const int blk = bid % nblk;
+    bid /= nblk;
+    const int kvh = bid % a.n_kv, seq = bid / a.n_kv;
+    const int pos0 = a.pos0[seq], kv_len = pos0 + a.S;
+    const int tb = (pos0 & ~31) + 32 * blk;
+    if (tb >= kv_len) return;
+    const size_t hb = (size_t)a.slot[seq] * a.n_kv + kvh;
+    const int lo = max(tb, pos0), hi = min(tb + 32, kv_len);
+    char* kb = (char*)a.kc + (hb * a.cap + tb) * AM_HD * ES;
+    char* vb = (char*)a.vc + (hb * a.cap + tb) * AM_HD * ES;
+    // the four rows of a wave's next step in one round trip
+    KvNew nv[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) nv[j] = load_kv_token(a, seq, kvh, pos0, min(max(tb + wid + 4 * j, lo), hi - 1));
+    if (lo > tb || hi < tb + 32) {
+        for (int i = tid * 16; i < KB; i += 256 * 16) {
+            *(u32x4v_t*)(st + i) = *(const u32x4v_t*)(kb + i);
+            *(u32x4v_t*)(st + KB + i) = *(const u32x4v_t*)(vb + i);
+        }
+        if (KVF == KV_INT8 && tid < 64)
+            scl[tid >> 5][tid & 31] = (tid < 32 ? a.ks : a.vs)[hb * a.cap + tb + (tid & 31)];
+        __syncthreads();
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const int r = wid + 4 * j;
+        if (tb + r < lo || tb + r >= hi) continue;
+#pragma unroll
+        for (int which = 0; which < 2; which++) {
+            const float v0 = nv[j].v[which][0], v1 = nv[j].v[which][1];
+            const int o0 = which == 0 ? (int)k_off(0, r, lane, 32, AM_HD, KVF) : (int)vt_off(0, lane, r, 32, AM_HD, KVF);
+            const int o1 = which == 0 ? (int)k_off(0, r, lane + 64, 32, AM_HD, KVF)
+                                      : (int)vt_off(0, lane + 64, r, 32, AM_HD, KVF);
+            if constexpr (KVF == KV_INT8) {
+                const float amax = wave_max_f32(fmaxf(fabsf(v0), fabsf(v1)));
+                const float sc = amax <= FLT_EPSILON ? 1.0f : amax / 127.0f;
+                st[which * KB + o0] = (int8_t)fminf(fmaxf(roundf(v0 / sc), -127.0f), 127.0f);
+                st[which * KB + o1] = (int8_t)fminf(fmaxf(roundf(v1 / sc), -127.0f), 127.0f);
+                if (lane == 0) scl[which][r] = __builtin_bit_cast(uint16_t, (_Float16)sc);
+            } else {
+                ((_Float16*)(st + which * KB))[o0] = (_Float16)v0;
+                ((_Float16*)(st + which * KB))[o1] = (_Float16)v1;
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = tid * 16; i < KB; i += 256 * 16) {
+        *(u32x4v_t*)(kb + i) = *(const u32x4v_t*)(st + i);
+        *(u32x4v_t*)(vb + i) = *(const u32x4v_t*)(st + KB + i);
+    }
+    if (KVF == KV_INT8 && tid < 64)
+        const_cast<uint16_t*>(tid < 32 ? a.ks : a.vs)[hb * a.cap + tb + (tid & 31)] = scl[tid >> 5][tid & 31];
+}
+
 // Flash-decode attention on MFMA for head_dim 128 and fp16 / INT8 caches.
 // Workgroup = (sequence, kv head, tile of <= 16 query rows, token chunk), 8 waves;
 // wave w takes the chunk's 32-token blocks w, w+8, ... (INT8: the blocks before the
@@ -453,7 +524,9 @@ __device__ __forceinline__ void frag_out_pair(const XFrag& fo, int orow, int oco
 // the lane of their row.  Softmax runs in base 2 (v_exp_f32).  With one chunk
 // the workgroup writes the output; otherwise chunk partials go out with
 // coherent 16-byte stores and the last workgroup of the group merges them.
-template <int KVF, int DEPTH, bool DMA>
+// PRE: the new positions are in the cache already (kv_append_kernel) and each query tile
+// reads only the blocks up to its last row's position.
+template <int KVF, int DEPTH, bool DMA, bool PRE>
 __global__ void __launch_bounds__(512) attn_mfma_kernel(AttnArgs a) {
     // dynamic LDS: the DMA block stages during the token loop, then the wave merge
     extern __shared__ __attribute__((aligned(1024))) char am_lds[];
@@ -480,7 +553,9 @@ __global__ void __launch_bounds__(512) attn_mfma_kernel(AttnArgs a) {
     const int QD = a.n_heads * AM_HD;
     const size_t hb = (size_t)sl * a.n_kv + kvh;
     const int t_begin = chunk * a.chunk;
-    const int t_end = min(kv_len, t_begin + a.chunk);
+    const int seen = PRE ? pos0 + (r0 + R - 1) / G + 1 : kv_len;  // tokens the tile's rows attend to
+    const int t_end = min(seen, t_begin + a.chunk);
+    const int lim0 = PRE ? pos0 + r0 / G : pos0;  // tokens up to here are seen by every row
     constexpr int STEP = 32 * AM_WAVES;
     int tb = t_begin + 32 * wid;
     const int t_chunk_last = (t_end - 1) & ~31;
@@ -507,27 +582,25 @@ __global__ void __launch_bounds__(512) attn_mfma_kernel(AttnArgs a) {
         lds_dma4<true>(vsr, st + 2 * KVB + 256, sc_voff, t * 2);
     };
     // DMA schedule: the blocks wholly before the new positions ("old" blocks) go round
-    // robin to the eight waves; the blocks holding new positions ("tail" blocks) come
-    // first in their wave's list, and that wave writes the new positions into its staged
-    // copy of the block (patch_tail) and stores the block back whole, so no wave waits
-    // for the cache append (a workgroup barrier after a byte-wise append held every wave
-    // until the appending waves' loads and stores came back).  One or two tail blocks
-    // (decode and verify) all go to wave AM_TAIL, which hands its last n_tail + AM_HAND
-    // old blocks to wave 0 (the oldest wave of the workgroup, whose stream ends first:
-    // issue arbitration favours it, and timestamps put its stream's end 9 us before the
-    // others' at B = 32).  More tail blocks (prompt chunks) go round robin like the old
-    // ones.  Wave wid's i-th block: tb_of(i); a wave issues no load past its last block.
-    const int tail_start = pos0 < t_end ? max(t_begin, pos0 & ~31) : t_end;
-    const int n_old = (tail_start - t_begin) >> 5, n_tail = (t_end - tail_start + 31) >> 5;
+    // robin to the eight waves; the one or two blocks holding new positions ("tail" blocks,
+    // S <= AM_DECODE_S) come first in the list of wave AM_TAIL, and that wave writes the new
+    // positions into its staged copy of the block (patch_tail) and stores the block back
+    // whole, so no wave waits for the cache append (a workgroup barrier after a byte-wise
+    // append held every wave until the appending waves' loads and stores came back).  It
+    // hands its last n_tail + AM_HAND old blocks to wave 0 (the oldest wave of the
+    // workgroup, whose stream ends first: issue arbitration favours it, and timestamps put
+    // its stream's end 9 us before the others' at B = 32).  Wave wid's i-th block: tb_of(i);
+    // a wave issues no load past its last block.  With PRE every block is an old one.
+    const int tail_start = !PRE && pos0 < t_end ? max(t_begin, pos0 & ~31) : max(t_begin, t_end);
+    const int n_old = (tail_start - t_begin + 31) >> 5, n_tail = PRE ? 0 : max(0, (t_end - tail_start + 31) >> 5);
     auto own = [&](int n, int w) { return n > w ? (n - w + AM_WAVES - 1) / AM_WAVES : 0; };
-    const bool solo = n_tail <= AM_SOLO;
-    const int t_old = own(n_old, AM_TAIL), n_moved = solo && n_tail > 0 ? min(n_tail + AM_HAND, t_old) : 0;
-    const int n_lead = solo ? (wid == AM_TAIL ? n_tail : 0) : own(n_tail, wid);  // tail blocks first
-    const int n_first = solo && wid == AM_TAIL ? t_old - n_moved : own(n_old, wid);  // strided old blocks
+    const int t_old = own(n_old, AM_TAIL), n_moved = n_tail > 0 ? min(n_tail + AM_HAND, t_old) : 0;
+    const int n_lead = wid == AM_TAIL ? n_tail : 0;  // tail blocks first
+    const int n_first = wid == AM_TAIL ? t_old - n_moved : own(n_old, wid);  // strided old blocks
     const int n_blk = n_lead + n_first + (wid == 0 ? n_moved : 0);
     auto tb_of = [&](int i) __attribute__((always_inline)) {
         i = min(i, n_blk - 1);
-        if (i < n_lead) return tail_start + 32 * (solo ? i : wid + AM_WAVES * i);
+        if (i < n_lead) return tail_start + 32 * i;
         i -= n_lead;
         if (i < n_first) return t_begin + 32 * (wid + AM_WAVES * i);
         return t_begin + 32 * (AM_TAIL + AM_WAVES * (t_old - n_moved + i - n_first));  // handed over
@@ -539,7 +612,7 @@ __global__ void __launch_bounds__(512) attn_mfma_kernel(AttnArgs a) {
     // block (ahead of the block loads in the memory pipeline); other rows are loaded
     // when their block is patched.
     const int first_new = max(t_begin, pos0);
-    const bool has_first = n_lead > 0 && (solo || wid == 0);
+    const bool has_first = !PRE && n_lead > 0;
     KvNew pre[4];
     if (DMA && has_first)
 #pragma unroll
@@ -598,7 +671,7 @@ __global__ void __launch_bounds__(512) attn_mfma_kernel(AttnArgs a) {
             if (n_blk > 1) issue(st0 + AM_STAGE, tb_of(1));
         }
     } else {
-        if (t_end > pos0) append_new_kv(a, seq, kvh, hb, pos0, t_begin, t_end);
+        if (!PRE && t_end > pos0) append_new_kv(a, seq, kvh, hb, pos0, t_begin, t_end);
     }
 
     // ---- this lane's query row (lr): Q^T B operand, hi/lo, dims 32*lg + 8*kk + slot ----
@@ -661,7 +734,7 @@ __global__ void __launch_bounds__(512) attn_mfma_kernel(AttnArgs a) {
         float mx = -INFINITY;
         // a block wholly inside the chunk and before every row's own position needs no mask
         // (wave-uniform: tb is the wave's block)
-        if (tb + 32 <= t_end && tb + 31 <= pos0) {
+        if (tb + 32 <= t_end && tb + 31 <= lim0) {
 #pragma unroll
             for (int idx = 0; idx < 8; idx++) {
                 float ksc = sc2;
@@ -728,7 +801,7 @@ __global__ void __launch_bounds__(512) attn_mfma_kernel(AttnArgs a) {
             if (i + 1 < n_blk) wait_vmcnt<NL>();
             else wait_vmcnt<0>();
             __atomic_signal_fence(__ATOMIC_SEQ_CST);
-            if (i < n_lead) patch_tail(cur_st, tb);
+            if (!PRE && i < n_lead) patch_tail(cur_st, tb);
             KvRaw<KVF> cur;
 #pragma unroll
             for (int ts = 0; ts < 2; ts++)
@@ -835,28 +908,40 @@ __global__ void __launch_bounds__(512) attn_mfma_kernel(AttnArgs a) {
     if (a.fo.buf) frag_out_pair(a.fo, orow, ocol, o4, q);
 }
 
+template <int KVF, bool DMA, bool PRE>
+static int launch_mfma_pre(const AttnArgs& a, int grid, hipStream_t stream) {
+    constexpr size_t merge_bytes = sizeof(float) * AM_WAVES * AM_ROWS * AM_REC;
+    constexpr size_t dma_bytes = DMA ? (size_t)AM_WAVES * 2 * AM_STAGE : 0;
+    constexpr size_t bytes = dma_bytes > merge_bytes ? dma_bytes : merge_bytes;
+    static bool attr = false;
+    if (!attr) {
+        if (note_error(hipFuncSetAttribute((const void*)attn_mfma_kernel<KVF, 1, DMA, PRE>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes)))
+            return 4;
+        attr = true;
+    }
+    launch_timed(attn_mfma_kernel<KVF, 1, DMA, PRE>, dim3(grid), dim3(512), (uint32_t)bytes, stream, a);
+    return note_error(hipGetLastError()) ? 4 : 0;
+}
+
+// Up to AM_DECODE_S rows per sequence (verify, replay, decode) the new positions lie in at
+// most two blocks and the kernel appends them itself: the append launch would cost such a
+// forward 8-10 us per layer where its attention takes 15-20.  Prompt chunks append first
+// and skip the blocks their rows do not see.
+template <int KVF, bool DMA>
+static int launch_mfma(const AttnArgs& a, int grid, hipStream_t stream) {
+    if (a.S <= AM_DECODE_S) return launch_mfma_pre<KVF, DMA, false>(a, grid, stream);
+    const int nblk = (a.S + 30) / 32 + 1;  // cache blocks that S positions can touch
+    launch_timed(kv_append_kernel<KVF>, dim3(a.nseq * a.n_kv * nblk), dim3(256), 0, stream, a, nblk);
+    return launch_mfma_pre<KVF, DMA, true>(a, grid, stream);
+}
+
 int launch_attention(const AttnArgs& a, hipStream_t stream) {
     const int grid = a.nseq * a.n_kv * a.ntiles * a.nchunks;
     (void)hipGetLastError();
     if ((a.kv_fmt == KV_INT8 || a.kv_fmt == KV_F16) && a.hd == AM_HD) {
         if (a.rows_per_tile > AM_ROWS || a.chunk % (32 * AM_WAVES) || a.nchunks > AM_MAXCH || a.cap % 32) return 3;
-        static bool attr = false;
-        constexpr size_t merge_bytes = sizeof(float) * AM_WAVES * AM_ROWS * AM_REC;
-        constexpr size_t dma_bytes = (size_t)AM_WAVES * 2 * AM_STAGE;
-        constexpr size_t i8_bytes = dma_bytes > merge_bytes ? dma_bytes : merge_bytes;
-        if (!attr) {
-            if (note_error(hipFuncSetAttribute((const void*)attn_mfma_kernel<KV_INT8, 1, true>,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)i8_bytes)) ||
-                note_error(hipFuncSetAttribute((const void*)attn_mfma_kernel<KV_F16, 1, false>,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)merge_bytes)))
-                return 4;
-            attr = true;
-        }
-        if (a.kv_fmt == KV_INT8)
-            launch_timed(attn_mfma_kernel<KV_INT8, 1, true>, dim3(grid), dim3(512), (uint32_t)i8_bytes, stream, a);
-        else
-            launch_timed(attn_mfma_kernel<KV_F16, 1, false>, dim3(grid), dim3(512), (uint32_t)merge_bytes, stream, a);
-        return note_error(hipGetLastError()) ? 4 : 0;
+        return a.kv_fmt == KV_INT8 ? launch_mfma<KV_INT8, true>(a, grid, stream) : launch_mfma<KV_F16, false>(a, grid, stream);
     }
     if (a.hd > AT_MAXHD || a.rows_per_tile > AT_MAXR || a.rows_per_tile <= 0) return 3;
     launch_timed(attn_kernel, dim3(grid), dim3(AT_THREADS), 0, stream, a);
