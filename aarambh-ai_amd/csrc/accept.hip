@@ -70,6 +70,7 @@ struct RowFilt {
     uint64_t kkey;  // top-k: logits with logit_key >= kkey are kept (0: all)
     uint64_t pkey;  // top-p: probabilities with prob_key >= pkey are kept (0: all)
     int topp;       // top-p applies
+    double iT, iS, iR2;  // reciprocals of T, S and R2 (div_fast)
 };
 
 // exp(l / T - mx) of element j (0 when top-k drops it or l / T is not finite):
@@ -87,6 +88,26 @@ __device__ __forceinline__ float filt_prob(const RowFilt& f, float l, int j) {
     if (!f.topp) return p0;
     if (!(p0 > 0.0f) || prob_key(p0, j) < f.pkey) return 0.0f;
     return p0 / f.R2;
+}
+
+// filt_exp and filt_prob without branches, for the producers of the scans: equal to them
+// unless `bad` is set.  (Each branch of the plain forms ends a basic block, and the scan's
+// elements then run one f64 chain after another instead of interleaved.)
+__device__ __forceinline__ float filt_exp_fast(const RowFilt& f, float l, int j, bool& bad) {
+    const bool keep = logit_key(l, j) >= f.kkey;
+    bool b = false;
+    const float m = div_fast(l, f.iT, b);
+    const bool fin = fabsf(m) < INFINITY;
+    const float e = expf_fast(fin ? m - f.mx : -200.0f, b);
+    bad = bad | (b & keep);
+    return keep & fin ? e : 0.0f;
+}
+__device__ __forceinline__ float filt_prob_fast(const RowFilt& f, float l, int j, bool& bad) {
+    const float p0 = div_fast(filt_exp_fast(f, l, j, bad), f.iS, bad);
+    if (!f.topp) return p0;
+    const bool keep = p0 > 0.0f && prob_key(p0, j) >= f.pkey;
+    const float p = div_fast(keep ? p0 : 0.0f, f.iR2, bad);
+    return p;
 }
 
 // Row statistics handed from stage 1 to the resolving workgroup (ACC_RS_WORDS words per row).
@@ -120,6 +141,9 @@ __device__ inline RowFilt rs_load(const uint32_t* w, float T) {
     f.kkey = (uint64_t)rs_get(w, RS_KKEY) | ((uint64_t)rs_get(w, RS_KKEY + 1) << 32);
     f.pkey = (uint64_t)rs_get(w, RS_PKEY) | ((uint64_t)rs_get(w, RS_PKEY + 1) << 32);
     f.topp = (int)rs_get(w, RS_TOPP);
+    f.iT = 1.0 / (double)T;
+    f.iS = 1.0 / (double)f.S;
+    f.iR2 = 1.0 / (double)f.R2;
     return f;
 }
 
@@ -133,9 +157,16 @@ struct SelShared {
     unsigned cnt, total;
 };
 
+// Windows of a scan chunk: plain sum, integer sum in ulps (-1: unusable) and its binade.
+struct ScanShared {
+    float wf[2 * ACC_WAVES];
+    int wi[2 * ACC_WAVES], we[2 * ACC_WAVES];
+};
+
 struct AccShared {
     SelShared sel;
     SeqScan scan;
+    ScanShared win;
     float red_f[ACC_WAVES], red_g[ACC_WAVES];
     int red_k[ACC_WAVES], red_i[ACC_WAVES];
     unsigned n;
@@ -304,37 +335,114 @@ __device__ __forceinline__ uint64_t select_desc(const KF& kf, const float* row, 
 // chunks of `chunk` values, double buffered (buf holds 2 * chunk floats): every wave
 // writes chunk 0, then wave 0 scans chunk c, carrying the running sum, while the
 // other waves write chunk c + 1 into the other half.
-template <int NR, class F>
-__device__ __forceinline__ SeqScan block_seq_scan(const float* r0, const float* r1, int n, float u, const F& f, float* buf,
-                                  int chunk, AccShared* sh) {
-    const int tid = threadIdx.x, wid = tid >> 6;
-    SeqScan st = seq_scan_init();
-    rows_foreach<NR>(r0, NR == 2 ? r1 : nullptr, min(chunk, n), [&](int i, float a, float b, bool valid) {
-        if (valid) buf[i] = f(a, b, i);
-    });
+//
+// Before the scan of a chunk all waves sum its windows of SCAN_WIN values: inside one binade
+// the running sum grows by the integer sum of RNE(x / ulp) (see seq_scan_wave), which does
+// not depend on the sum itself, only on its binade.  The binade at each window's start is
+// predicted from plain f32 sums; the scan uses a window's integer sum only where the
+// running sum is in that binade and stays in it, no element is special and the draw u is not
+// reached, and walks the window itself otherwise (the windows that cross a binade: about one
+// for each doubling of the sum).  So the prediction decides the time and never the result.
+// What bounds it now is the producing: with two exact exponentials and five exact quotients per
+// residual, one workgroup writes an 8192-value chunk in 6-12 us, against 3-5 us for scanning
+// it (10-15 us for the first chunk, whose sum doubles every few values).  32 sequences x 9
+// rows of 32 000 logits at temperature 0.8: 254 us before the window sums, the branch-free
+// producers and the parallel acceptance probabilities, 232 us with them.
+static_assert(ACC_CHUNK <= 2 * ACC_WAVES * SCAN_WIN, "two windows per wave");
+typedef __attribute__((address_space(3))) ScanShared lds_scan;
+__device__ __noinline__ static void scan_windows(lds_cfloat* buf, int m, float s0, lds_scan* sh) {
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float x[2][8];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const int win = wid + ACC_WAVES * q;
+        scan_load(buf + win * SCAN_WIN, m - win * SCAN_WIN, x[q]);
+        float t = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 8; k++) t += x[q][k];
+        t = wave_sum_f32(t);
+        if (lane == 0) sh->wf[win] = t;
+    }
     __syncthreads();
-    for (int c0 = 0; c0 < n; c0 += chunk) {
-        const int m = min(chunk, n - c0);
-        float* cur = buf + ((c0 / chunk) & 1) * chunk;
-        if (wid == 0) {
-            seq_scan_wave(cur, m, u, c0, st);
-        } else if (c0 + chunk < n) {
-            const int c1 = c0 + chunk, m1 = min(chunk, n - c1);
-            float* nxt = buf + (((c0 / chunk) + 1) & 1) * chunk;
-            constexpr int NT = ACC_THREADS - 64, U = 4;
-            for (int i0 = tid - 64; i0 < m1; i0 += U * NT) {
-                float va[U], vb[U];
+    // lane l of the first 2 ACC_WAVES: predicted sum at the start of window l
+    float incl = lane < 2 * ACC_WAVES ? sh->wf[lane] : 0.0f;
+    const float own = incl;
+#pragma unroll
+    for (int d = 1; d < 2 * ACC_WAVES; d <<= 1) {
+        const float t = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += t;
+    }
+    const float start = s0 + (incl - own);
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const int win = wid + ACC_WAVES * q;
+        const int eb = (int)((__float_as_uint(readlane_f32(start, win)) >> 23) & 0xFF);
+        bool bad;
+        const int total = wave_incl_scan_dpp(scan_increments(x[q], 150 - eb, bad));
+        const bool any = __ballot(bad) != 0ull || eb < SCAN_MIN_EB || eb == 255;
+        if (lane == 63) {
+            sh->wi[win] = any ? -1 : total;
+            sh->we[win] = eb;
+        }
+    }
+    __syncthreads();
+}
+
+//
+// The scanned function comes in two forms of equal value: f(a, b, j, bad) without branches,
+// and g(a, b, j), which decides where f sets bad.
+template <int NR, class F, class G>
+__device__ __forceinline__ SeqScan block_seq_scan(const float* r0, const float* r1, int n, float u, const F& f, const G& g,
+                                  float* buf, int chunk, AccShared* sh) {
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    SeqScan st = seq_scan_init();
+    if (tid == 0) sh->scan.s = 0.0f;
+    // step -1 writes chunk 0; step c >= 0 scans chunk c on wave 0 while the others write c + 1
+    for (int c = -1; c < 0 || c * chunk < n; c++) {
+        const int m = min(chunk, n - c * chunk);
+        float* cur = buf + (c & 1) * chunk;
+        if (c >= 0) scan_windows((lds_cfloat*)cur, m, sh->scan.s, (lds_scan*)&sh->win);
+        if (c >= 0 && wid == 0) {
+            const int wi = lane < 2 * ACC_WAVES ? sh->win.wi[lane] : -1, we = lane < 2 * ACC_WAVES ? sh->win.we[lane] : 0;
+            __builtin_amdgcn_s_setprio(3);  // the serial chain goes ahead of the producers on its SIMD
+            st = seq_scan_chunk((lds_cfloat*)cur, m, u, c * chunk, st, wi, we);
+            __builtin_amdgcn_s_setprio(0);
+            if (tid == 0) sh->scan.s = st.s;
+        } else if ((c + 1) * chunk < n) {
+            const int c1 = (c + 1) * chunk, m1 = min(chunk, n - c1);
+            float* nxt = buf + ((c + 1) & 1) * chunk;
+            const int t0 = c < 0 ? tid : tid - 64, nt = c < 0 ? ACC_THREADS : ACC_THREADS - 64;
+            // the next step's loads are in flight while this step's values are computed
+            constexpr int U = 4;
+            float va[U], vb[U];
+            auto load = [&](int i0) __attribute__((always_inline)) {
 #pragma unroll
                 for (int q = 0; q < U; q++) {
-                    const int i = i0 + q * NT;
-                    va[q] = i < m1 ? r0[c1 + i] : 0.f;
-                    vb[q] = (NR == 2 && i < m1) ? r1[c1 + i] : 0.f;
+                    const int i = c1 + min(i0 + q * nt, m1 - 1);
+                    va[q] = r0[i];
+                    vb[q] = NR == 2 ? r1[i] : 0.f;
                 }
+            };
+            if (t0 < m1) load(t0);
+#pragma unroll 1
+            for (int i0 = t0; i0 < m1; i0 += U * nt) {
+                float wa[U], wb[U];
 #pragma unroll
                 for (int q = 0; q < U; q++) {
-                    const int i = i0 + q * NT;
-                    if (i < m1) nxt[i] = f(va[q], vb[q], c1 + i);
+                    wa[q] = va[q];
+                    wb[q] = vb[q];
                 }
+                load(i0 + U * nt);
+                float y[U];
+                bool bad = false;
+#pragma unroll
+                for (int q = 0; q < U; q++) y[q] = f(wa[q], wb[q], c1 + i0 + q * nt, bad);
+                if (bad)
+#pragma unroll
+                    for (int q = 0; q < U; q++) y[q] = g(wa[q], wb[q], c1 + i0 + q * nt);
+#pragma unroll
+                for (int q = 0; q < U; q++)
+                    if (i0 + q * nt < m1) nxt[i0 + q * nt] = y[q];
             }
         }
         __syncthreads();
@@ -727,6 +835,7 @@ __device__ inline void row_filter_topk(float top_p, int n, float* buf, AccShared
     for (int i = tid; i < n; i += ACC_THREADS) vals[i] = filt_exp(fe, surv_logit(keys[i]), surv_index(keys[i]));
     __syncthreads();
     f.S = seq_sum_w0(vals, n, sh);
+    f.iS = 1.0 / (double)f.S;
     if (!(f.S > 0.0f) || !isfinite(f.S)) {
         status = 1;
         return;
@@ -789,6 +898,7 @@ __device__ inline void row_filter_topk(float top_p, int n, float* buf, AccShared
     }
     __syncthreads();
     f.R2 = seq_sum_w0(kept, n, sh);
+    f.iR2 = 1.0 / (double)f.R2;
     flags |= (uint32_t)sh->ib[7];
     __syncthreads();
     if (!(f.R2 > 0.0f) || !isfinite(f.R2)) status = 1;
@@ -806,6 +916,8 @@ __device__ __forceinline__ void row_filter(const float* row, int V, float T, int
     f.pkey = 0;
     f.R2 = 1.0f;
     f.S = 1.0f;
+    f.iT = 1.0 / (double)T;
+    f.iS = f.iR2 = 1.0;
     f.mx = 0.0f;
     f.topp = (top_p > 0.0f && top_p < 1.0f) ? 1 : 0;
     flags = 0;
@@ -834,15 +946,26 @@ __device__ __forceinline__ void row_filter(const float* row, int V, float T, int
         f.kkey = select_desc(kf, row, V, top_k, ~0ull, sh, &tot);
     }
     // ---- max of the finite masked logits ----
+    // l / T grows with l, so the max of the finite l / T is that of the largest finite l, unless
+    // dividing by T < 1 makes that one infinite
     float mx = -INFINITY;
     const uint64_t kk = f.kkey;
-    rows_foreach<1>(row, nullptr, V, [&](int j, float l, float, bool valid) {
-        if (valid && logit_key(l, j) >= kk) {
-            const float m = l / T;
-            if (isfinite(m)) mx = fmaxf(mx, m);
-        }
-    });
-    mx = block_max(mx, sh);
+    if (kk == 0) {
+        rows_foreach<1>(row, nullptr, V, [&](int, float l, float, bool valid) {
+            if (valid && fabsf(l) < INFINITY) mx = fmaxf(mx, l);
+        });
+        mx = block_max(mx, sh) / T;
+    }
+    if (kk != 0 || mx == INFINITY) {
+        mx = -INFINITY;
+        rows_foreach<1>(row, nullptr, V, [&](int j, float l, float, bool valid) {
+            if (valid && logit_key(l, j) >= kk) {
+                const float m = l / T;
+                if (isfinite(m)) mx = fmaxf(mx, m);
+            }
+        });
+        mx = block_max(mx, sh);
+    }
     if (!(mx > -INFINITY)) {  // "all logits are non-finite" (sampler.rs:286-288)
         status = 1;
         return;
@@ -851,8 +974,10 @@ __device__ __forceinline__ void row_filter(const float* row, int V, float T, int
     // ---- softmax normaliser: exact sequential sum in index order ----
     const RowFilt fe = f;
     const SeqScan s1 = block_seq_scan<1>(
-        row, nullptr, V, -1.0f, [&](float a, float, int j) { return filt_exp(fe, a, j); }, buf, chunk, sh);
+        row, nullptr, V, -1.0f, [&](float a, float, int j, bool& bad) { return filt_exp_fast(fe, a, j, bad); },
+        [&](float a, float, int j) { return filt_exp(fe, a, j); }, buf, chunk, sh);
     f.S = s1.s;
+    f.iS = 1.0 / (double)f.S;
     if (!(f.S > 0.0f) || !isfinite(f.S)) {
         status = 1;
         return;
@@ -901,7 +1026,7 @@ __device__ __forceinline__ void row_filter(const float* row, int V, float T, int
         if (wid == 0) {
             SeqScan st = seq_scan_init();
             st.s = carry;
-            seq_scan_wave(vals, n, top_p, 0, st);
+            st = seq_scan_chunk((lds_cfloat*)vals, n, top_p, 0, st, -1, 0);
             if (tid == 0) sh->scan = st;
         }
         __syncthreads();
@@ -922,12 +1047,17 @@ __device__ __forceinline__ void row_filter(const float* row, int V, float T, int
     const RowFilt fr = f;
     const SeqScan s2 = block_seq_scan<1>(
         row, nullptr, V, -1.0f,
+        [&](float a, float, int j, bool& bad) {
+            const float p0 = div_fast(filt_exp_fast(fr, a, j, bad), fr.iS, bad);
+            return (p0 > 0.0f && prob_key(p0, j) >= fr.pkey) ? p0 : 0.0f;
+        },
         [&](float a, float, int j) {
             const float p0 = filt_exp(fr, a, j) / fr.S;
             return (p0 > 0.0f && prob_key(p0, j) >= fr.pkey) ? p0 : 0.0f;
         },
         buf, chunk, sh);
     f.R2 = s2.s;
+    f.iR2 = 1.0 / (double)f.R2;
     if (!(f.R2 > 0.0f) || !isfinite(f.R2)) status = 1;
 }
 
@@ -1044,6 +1174,24 @@ __global__ void __launch_bounds__(ACC_THREADS) __attribute__((amdgpu_waves_per_e
             u_s[tid] = rng_f32(key, (a.word_offsets ? a.word_offsets[b] : 0ull) + tid);
         }
     }
+    // ... and proposal d's probabilities, so that the decisions below run from LDS instead of
+    // through one chain of row statistics, token and logit loads after another
+    auto proposal = [&](int i, float& p, float& q, uint32_t& fl, int& st) {
+        const uint32_t* wt = rs0 + i * ACC_RS_WORDS;
+        const uint32_t* wd = rsd0 + i * ACC_RS_WORDS;
+        fl = rs_get(wt, RS_FLAGS) | rs_get(wd, RS_FLAGS);
+        st = (int)(rs_get(wt, RS_STATUS) | rs_get(wd, RS_STATUS));
+        p = q = 0.0f;
+        const uint32_t x = a.draft_tokens[(size_t)b * a.K + i];
+        if (st == 0 && x < (uint32_t)V) {
+            p = filt_prob(rs_load(wt, T), trow0[(size_t)i * V + x], (int)x);
+            q = filt_prob(rs_load(wd, T), drow0[(size_t)i * V + x], (int)x);
+        }
+    };
+    __shared__ float p_s[64], q_s[64];
+    __shared__ uint32_t fl_s[64];
+    __shared__ int st_s[64];
+    if (par_u && tid < np) proposal(tid, p_s[tid], q_s[tid], fl_s[tid], st_s[tid]);
     __syncthreads();
 
     if (tid == 0) {
@@ -1061,19 +1209,22 @@ __global__ void __launch_bounds__(ACC_THREADS) __attribute__((amdgpu_waves_per_e
                 rej = i;
                 break;
             }
-            const uint32_t* wt = rs0 + i * ACC_RS_WORDS;
-            const uint32_t* wd = rsd0 + i * ACC_RS_WORDS;
-            flags |= rs_get(wt, RS_FLAGS) | rs_get(wd, RS_FLAGS);
-            if (rs_get(wt, RS_STATUS) | rs_get(wd, RS_STATUS)) {
+            float p, q;
+            uint32_t fl;
+            int st;
+            if (par_u) {
+                p = p_s[i];
+                q = q_s[i];
+                fl = fl_s[i];
+                st = st_s[i];
+            } else {
+                proposal(i, p, q, fl, st);
+            }
+            flags |= fl;
+            if (st) {
                 status = 1;
                 rej = i;
                 break;
-            }
-            const uint32_t x = a.draft_tokens[(size_t)b * a.K + i];
-            float p = 0.0f, q = 0.0f;
-            if ((int)x < V) {
-                p = filt_prob(rs_load(wt, T), trow0[(size_t)i * V + x], (int)x);
-                q = filt_prob(rs_load(wd, T), drow0[(size_t)i * V + x], (int)x);
             }
             if (!(q > 0.0f)) {
                 rej = i;
@@ -1147,19 +1298,27 @@ __global__ void __launch_bounds__(ACC_THREADS) __attribute__((amdgpu_waves_per_e
                 const float d = filt_prob(ft, lt, j) - filt_prob(fd, ld, j);
                 return d > 0.0f ? d : 0.0f;
             };
-            const SeqScan m = block_seq_scan<2>(tl, dl, V, -1.0f, resid, lds, chunk, &sh);
+            auto resid_fast = [&](float lt, float ld, int j, bool& bad) {
+                const float d = filt_prob_fast(ft, lt, j, bad) - filt_prob_fast(fd, ld, j, bad);
+                return d > 0.0f ? d : 0.0f;
+            };
+            const SeqScan m = block_seq_scan<2>(tl, dl, V, -1.0f, resid_fast, resid, lds, chunk, &sh);
             const float R = m.s;
             if (!isfinite(R) || R <= FLT_EPSILON) {
                 status = 1;
             } else {
+                const double iR = 1.0 / (double)R;
                 cdf = block_seq_scan<2>(
-                    tl, dl, V, u, [&](float lt, float ld, int j) { return resid(lt, ld, j) / R; }, lds, chunk, &sh);
+                    tl, dl, V, u,
+                    [&](float lt, float ld, int j, bool& bad) { return div_fast(resid_fast(lt, ld, j, bad), iR, bad); },
+                    [&](float lt, float ld, int j) { return resid(lt, ld, j) / R; }, lds, chunk, &sh);
             }
         } else {
             const RowFilt ft = rs_load(rs0 + np * ACC_RS_WORDS, T);
             cdf = block_seq_scan<1>(
-                trow0 + (size_t)np * V, nullptr, V, u, [&](float lt, float, int j) { return filt_prob(ft, lt, j); },
-                lds, chunk, &sh);
+                trow0 + (size_t)np * V, nullptr, V, u,
+                [&](float lt, float, int j, bool& bad) { return filt_prob_fast(ft, lt, j, bad); },
+                [&](float lt, float, int j) { return filt_prob(ft, lt, j); }, lds, chunk, &sh);
         }
         if (status == 0) {
             if (cdf.cross < 0) {  // no partial sum reaches the draw: the last index (sampler.rs:346)

@@ -38,6 +38,45 @@ __device__ __forceinline__ int32_t total_key(float f) {
 // itself misrounds; those show up as flagged near-ties, never silently.
 __device__ __forceinline__ float expf_rn(float x) { return (float)exp((double)x); }
 
+// The same value without branches, or `bad` set (then expf_rn decides).  For |x| < 87 (a
+// normal f32 result) a Taylor polynomial of degree 11 on |r| <= ln 2 / 2, r = x - k ln 2,
+// gives e^x within 2^-45 relative: r^12 / 12! is below 2^-47 and the f64 roundings add a few
+// 2^-52.  Rounding it to f32 equals rounding any value within that distance, unless it lies
+// next to a midpoint of two f32 values: within 2^-42 of one (one value in 2^18) it is bad.
+// Below -104 the result is 0 (e^-104 < 2^-150).  All 2^32 inputs compared with expf_rn.
+__device__ __forceinline__ float expf_fast(float x, bool& bad) {
+    const double xd = (double)x;
+    const double k = __builtin_rint(xd * 1.4426950408889634);
+    const double r = fma(-k, 0.6931471805599453, xd);
+    double p = 1.0 / 39916800.0;
+    p = fma(p, r, 1.0 / 3628800.0);
+    p = fma(p, r, 1.0 / 362880.0);
+    p = fma(p, r, 1.0 / 40320.0);
+    p = fma(p, r, 1.0 / 5040.0);
+    p = fma(p, r, 1.0 / 720.0);
+    p = fma(p, r, 1.0 / 120.0);
+    p = fma(p, r, 1.0 / 24.0);
+    p = fma(p, r, 1.0 / 6.0);
+    p = fma(p, r, 0.5);
+    p = fma(p, r, 1.0);
+    p = fma(p, r, 1.0);
+    // the 29 bits below f32 precision, measured from the midpoint (2^28) in units of 2^-52
+    const uint32_t d = ((uint32_t)__double2loint(p) & 0x1FFFFFFFu) - (0x10000000u - 1024u);
+    const bool zero = x < -104.0f;
+    bad = bad | ((!(fabsf(x) < 87.0f) | (d <= 2048u)) & !zero);
+    return zero ? 0.0f : (float)__builtin_ldexp(p, (int)k);
+}
+
+// x / d, correctly rounded, with inv = 1 / (double)d and no branch.  The quotient of two 24-bit
+// numbers lies at least 2^-49 (relative) from every midpoint of two f32 values, and x * inv
+// in f64 within 2^-51.9 of it, so both round to the same f32.  `bad` is set for results near
+// the subnormal range (where f32 has fewer bits) and NaN: then x / d decides.
+__device__ __forceinline__ float div_fast(float x, double inv, bool& bad) {
+    const float y = (float)((double)x * inv);
+    bad = bad | !((fabsf(y) > 1e-30f) | (x == 0.0f));
+    return y;
+}
+
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 __device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
     uint32_t x = __float_as_uint(f);
@@ -210,9 +249,11 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
 // Method: while s stays inside one binade [2^e, 2^(e+1)), every partial sum
 // is an integer multiple of ulp(s), and fl(s + x) = s + ulp * RNE(x / ulp)
 // unless x / ulp has fraction exactly 1/2 (a tie, decided by parity).  So the
-// wave turns 512 elements at a time into integer increments, scans them, and
-// stops at the first element that leaves the binade or ties; that element is
-// added with a real f32 add and the scan restarts after it.
+// wave turns 512 elements (8 consecutive ones per lane, held in registers) into integer
+// increments and scans them over the lanes.  The lanes before the first one that
+// leaves the binade, holds a tie or reaches u are taken at once; that lane's 8 elements
+// are added one after another with real f32 adds.  The lanes after it keep their
+// increments if the sum is still in the binade, and are turned again otherwise.
 // ---------------------------------------------------------------------------
 struct SeqScan {
     float s;         // running sum
@@ -245,236 +286,145 @@ __device__ __forceinline__ float readlane_f32(float x, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
 }
 
-// Elements added one at a time after the sum first becomes non-zero (see below).
-constexpr int SCAN_SCALAR = 64;
-__device__ __forceinline__ void seq_scan_wave(const float* v, int n, float u, int gbase, SeqScan& st) {
-    constexpr int E = 8;  // consecutive elements per lane in the binade fast path (512 per step)
+constexpr int SCAN_WIN = 512;  // elements per window: 8 per lane
+
+// LDS pointers as such: the scans are functions of their own (one copy of their code for all
+// callers), where a plain pointer would be read through the flat path.
+typedef __attribute__((address_space(3))) const float lds_cfloat;
+typedef __attribute__((address_space(3))) const float4_t lds_cfloat4;
+
+// The lane's 8 elements of the window v[0..n), n <= SCAN_WIN (0 past the end).
+__device__ __forceinline__ void scan_load(lds_cfloat* v, int n, float (&x)[8]) {
+    const int base = 8 * (threadIdx.x & 63);
+    if (base + 8 <= n) {
+        const float4_t a = *(lds_cfloat4*)(v + base), b = *(lds_cfloat4*)(v + base + 4);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            x[k] = a[k];
+            x[4 + k] = b[k];
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 8; k++) x[k] = base + k < n ? v[base + k] : 0.0f;
+    }
+}
+
+// Sums of at least 2^-103 (biased exponent 24 up) are scanned by increments: the scale 2^sft
+// is then a normal f32 and x * 2^sft is exact or far above 2^24.
+constexpr int SCAN_MIN_EB = 24;
+__device__ __forceinline__ float scan_pow2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
+
+// Sum of the lane's increments RNE(x / ulp), ulp = 2^-sft.  `special`: an element is a tie or
+// not a finite value in [0, 2^24) ulps (its bit pattern, read as unsigned, is at or above
+// that of 2^24: also negative values and NaN), or the sum leaves any binade.
+__device__ __forceinline__ int scan_increments(const float (&x)[8], int sft, bool& special) {
+    const float scale = scan_pow2(sft);
+    int lsum = 0;
+    float dmax = 0.0f;
+    uint32_t bmax = 0u;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const float c = x[k] * scale;
+        const float rr = __builtin_rintf(c);
+        dmax = fmaxf(dmax, fabsf(c - rr));
+        bmax = max(bmax, __float_as_uint(c));
+        lsum += (int)rr;
+    }
+    special = bmax >= 0x4B800000u || dmax == 0.5f || lsum >= 16777216;
+    return special ? 0 : lsum;
+}
+
+// Continues st over one window (x from scan_load, n elements, the first one index gbase).
+__device__ __forceinline__ void scan_window(const float (&x)[8], int n, float u, int gbase, SeqScan& st) {
     const int lane = threadIdx.x & 63;
+    const int lanes = (n + 7) >> 3;
     float s = st.s;
-    int pos = 0;
-    int cross = st.cross;
-    float s_at = st.s_at, s_before = st.s_before;
-    const bool want = u >= 0.0f;
-    int scal = 0;  // elements still to add one at a time
-    while (pos < n) {
-        if (scal > 0) {
-            // Plain f32 adds in element order (64 loaded per round trip, four added per
-            // crossing check).  Used for the first SCAN_SCALAR elements after the sum
-            // becomes non-zero, where the sum still doubles every few elements and the
-            // binade windows would restart at almost every element.
-            const int cnt = min(64, min(scal, n - pos));
-            const float xv = lane < cnt ? v[pos + lane] : 0.0f;  // lanes past cnt add 0: no change
-            for (int i = 0; i < cnt; i += 4) {
-                const float x0 = readlane_f32(xv, i), x1 = readlane_f32(xv, i + 1);
-                const float x2 = readlane_f32(xv, i + 2), x3 = readlane_f32(xv, i + 3);
-                const float s0 = s + x0, s1 = s0 + x1, s2 = s1 + x2, s3 = s2 + x3;
-                if (want && cross < 0 && (u <= s0 || u <= s1 || u <= s2 || u <= s3)) {
-                    // the first of the four partial sums to reach u (a padding lane repeats
-                    // the last real sum, so the first one found is a real element)
-                    const int k = u <= s0 ? 0 : u <= s1 ? 1 : u <= s2 ? 2 : 3;
-                    cross = gbase + pos + i + k;
-                    s_at = k == 0 ? s0 : k == 1 ? s1 : k == 2 ? s2 : s3;
-                    s_before = k == 0 ? s : k == 1 ? s0 : k == 2 ? s1 : s2;
+    int from = 0;  // first lane not yet added
+    // the elements of lane `stop`, one f32 add each
+    auto add_lane = [&](int stop) __attribute__((always_inline)) {
+        if (u >= 0.0f && st.cross < 0) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const float before = s;
+                s = before + readlane_f32(x[k], stop);
+                if (st.cross < 0 && u <= s && 8 * stop + k < n) {
+                    st.cross = gbase + 8 * stop + k;
+                    st.s_at = s;
+                    st.s_before = before;
                 }
-                s = s3;
-            }
-            pos += cnt;
-            scal -= cnt;
-            continue;
-        }
-        if (s == 0.0f) {
-            // Zeros keep s at 0 (0 + 0 = 0); the first non-zero element x gives s = x.
-            const int base = pos + 4 * lane;
-            float x[4];
-#pragma unroll
-            for (int k = 0; k < 4; k++) x[k] = (base + k < n) ? v[base + k] : 0.0f;
-            int fnz = 4;
-#pragma unroll
-            for (int k = 3; k >= 0; k--)
-                if (base + k < n && x[k] != 0.0f) fnz = k;
-            unsigned long long m = __ballot(fnz < 4);
-            if (want && cross < 0 && u <= 0.0f) {
-                cross = gbase + pos;
-                s_at = 0.0f;
-                s_before = 0.0f;
-            }
-            if (m == 0ull) {
-                pos += 256;
-                continue;
-            }
-            const int bl = __ffsll((long long)m) - 1;
-            const int t = pos + 4 * bl + __builtin_amdgcn_readlane(fnz, bl);
-            s = v[t];
-            if (want && cross < 0 && u <= s) {
-                cross = gbase + t;
-                s_at = s;
-                s_before = 0.0f;
-            }
-            pos = t + 1;
-            scal = SCAN_SCALAR;
-            continue;
-        }
-        const uint32_t bits = __float_as_uint(s);
-        const int eb = (int)((bits >> 23) & 0xFF);
-        if (eb == 0) {
-            // subnormal running sum: one scalar step
-            const float xt = v[pos];
-            const float sp = s;
-            s = s + xt;
-            if (want && cross < 0 && u <= s) {
-                cross = gbase + pos;
-                s_at = s;
-                s_before = sp;
-            }
-            pos++;
-            continue;
-        }
-        const int sh = 150 - eb;                               // x / ulp(s) == ldexp(x, sh)
-        const int ns = (int)((bits & 0x7FFFFFu) | 0x800000u);  // s / ulp(s)
-        // window [w0, w0 + 64 E) aligned to 4 elements; elements below pos count as 0
-        const int w0 = pos & ~3;
-        const int base = w0 + E * lane;
-        float x[E];
-        if (base + E <= n && base >= pos) {
-#pragma unroll
-            for (int c = 0; c < E / 4; c++) {
-                const float4_t q = *(const float4_t*)(v + base + 4 * c);
-                x[4 * c] = q[0];
-                x[4 * c + 1] = q[1];
-                x[4 * c + 2] = q[2];
-                x[4 * c + 3] = q[3];
             }
         } else {
 #pragma unroll
-            for (int k = 0; k < E; k++) {
-                const int i = base + k;
-                x[k] = (i >= pos && i < n) ? v[i] : 0.0f;
-            }
+            for (int k = 0; k < 8; k++) s += readlane_f32(x[k], stop);
         }
-        // r = RNE(c) for c = x / ulp.  An element is special when c is not a finite value
-        // in [0, 2^24) (its bit pattern, read as unsigned, is at or above that of 2^24:
-        // also negative values and NaN) or is a tie (|c - RNE(c)| == 1/2).  The lane
-        // tests both once over its E elements with vector max operations, and only a
-        // flagged lane marks its elements one by one (special elements become 2^24).
-        int r[E];
-        bool special = false;
-        int lsum = 0;
-        float dmax = 0.0f;
-        uint32_t bmax = 0u;
+        from = stop + 1;
+    };
+    while (from < lanes) {
+        const uint32_t bits = (uint32_t)__builtin_amdgcn_readfirstlane(__float_as_int(s));
+        const int eb = (int)(bits >> 23);
+        if (eb < SCAN_MIN_EB || eb >= 255) {
+            // zero or tiny sum (or none): lanes of zeros leave a zero sum as it is
+            uint32_t any = 0u;
 #pragma unroll
-        for (int k = 0; k < E; k++) {
-            const float c = ldexpf(x[k], sh);
-            const float rr = __builtin_rintf(c);
-            dmax = fmaxf(dmax, fabsf(c - rr));
-            bmax = max(bmax, __float_as_uint(c));
-            r[k] = (int)rr;
-            lsum += r[k];
+            for (int k = 0; k < 8; k++) any |= __float_as_uint(x[k]) << 1;
+            const unsigned long long m = __ballot(lane >= from && any != 0u);
+            const bool skip = s == 0.0f && !(u >= 0.0f && u <= 0.0f && st.cross < 0);
+            const int stop = skip ? (m ? __ffsll((long long)m) - 1 : 64) : from;
+            if (stop >= lanes) break;
+            add_lane(stop);
+            continue;
         }
-        if (bmax >= 0x4B800000u || dmax == 0.5f) {
-            special = true;
-            lsum = 0;
-#pragma unroll
-            for (int k = 0; k < E; k++) {
-                const float c = ldexpf(x[k], sh);
-                const float rr = __builtin_rintf(c);
-                const bool sp = !(__float_as_uint(c) < 0x4B800000u) || (fabsf(c - rr) == 0.5f);
-                r[k] = sp ? 16777216 : (int)rr;
-                lsum += r[k];
-            }
-        }
-        if (special || lsum > 16777217) lsum = 16777217;  // past the binade anyway; keeps the scan in range
+        const int sft = 150 - eb;                            // x / ulp(s) == x * 2^sft
+        const float ulp = scan_pow2(-sft);
+        int base = (int)((bits & 0x7FFFFFu) | 0x800000u);    // s / ulp(s), less the increments of lanes < from
+        bool special;
+        int lsum = scan_increments(x, sft, special);
+        if (lane < from) lsum = 0;
         const int incl = wave_incl_scan_dpp(lsum);
-        // Fast path: no element is special and the window ends inside the binade, and no
-        // partial sum of the window reaches u (sums only grow, so each lane's end value
-        // decides): the window advances without walking its elements.
-        {
-            const int lane_end = ns + incl;
-            const bool lane_bad = special || lane_end >= 16777216;
-            const bool lane_cross = want && cross < 0 && u <= ldexpf((float)lane_end, -sh);
-            if (__ballot(lane_bad || lane_cross) == 0ull) {
-                s = ldexpf((float)(ns + __builtin_amdgcn_readlane(incl, 63)), -sh);
-                pos = w0 + 64 * E;
-                continue;
+        for (;;) {
+            const int end = base + incl;
+            const bool halt = special || end >= 16777216 ||
+                              (u >= 0.0f && st.cross < 0 && u <= (float)end * ulp);
+            const unsigned long long m = __ballot(halt && lane >= from);
+            const int stop = m ? __ffsll((long long)m) - 1 : 64;
+            s = (float)(stop == 64 ? __builtin_amdgcn_readlane(end, 63)
+                                   : __builtin_amdgcn_readlane(end - lsum, stop)) * ulp;
+            if (stop >= lanes) {
+                from = lanes;
+                break;
             }
-        }
-        int run = ns + incl - lsum;
-        int first_bad = E, first_cross = E, run_bad = 0;
-        float cs_at = 0.0f, cs_before = 0.0f;
-        // walk the lane's elements with predication only (no early exit), so the loop
-        // unrolls and r[] stays in registers
-#pragma unroll
-        for (int k = 0; k < E; k++) {
-            const int rk = run + r[k];
-            const bool live = first_bad == E;
-            if (live && (r[k] >= 16777216 || rk >= 16777216)) {
-                first_bad = k;
-                run_bad = run;
-            }
-            if (want && first_bad == E && first_cross == E && r[k] > 0) {
-                const float sk = ldexpf((float)rk, -sh);
-                if (u <= sk) {
-                    first_cross = k;
-                    cs_at = sk;
-                    cs_before = ldexpf((float)run, -sh);
-                }
-            }
-            if (first_bad == E) run = rk;
-        }
-        const unsigned long long badm = __ballot(first_bad < E);
-        const int bad_lane = badm ? (__ffsll((long long)badm) - 1) : 64;
-        const unsigned long long lanes_ok = bad_lane >= 64 ? ~0ull : ((1ull << bad_lane) | ((1ull << bad_lane) - 1ull));
-        const unsigned long long cm = __ballot(first_cross < E) & lanes_ok;
-        if (want && cross < 0 && cm) {
-            const int cl = __ffsll((long long)cm) - 1;
-            cross = gbase + w0 + E * cl + __builtin_amdgcn_readlane(first_cross, cl);
-            s_at = readlane_f32(cs_at, cl);
-            s_before = readlane_f32(cs_before, cl);
-        }
-        if (bad_lane == 64) {
-            s = ldexpf((float)(ns + __builtin_amdgcn_readlane(incl, 63)), -sh);
-            pos = w0 + 64 * E;
-        } else {
-            const int t = w0 + E * bad_lane + __builtin_amdgcn_readlane(first_bad, bad_lane);
-            const float sp = ldexpf((float)__builtin_amdgcn_readlane(run_bad, bad_lane), -sh);
-            const float xt = v[t];
-            s = sp + xt;
-            if (want && cross < 0 && u <= s) {
-                cross = gbase + t;
-                s_at = s;
-                s_before = sp;
-            }
-            pos = t + 1;
+            add_lane(stop);
+            const uint32_t nb = (uint32_t)__builtin_amdgcn_readfirstlane(__float_as_int(s));
+            if (from >= lanes || (int)(nb >> 23) != eb) break;
+            base = (int)((nb & 0x7FFFFFu) | 0x800000u) - __builtin_amdgcn_readlane(incl, stop);
         }
     }
     st.s = s;
-    st.cross = cross;
-    st.s_at = s_at;
-    st.s_before = s_before;
 }
 
-// One-shot form over v[0..n): total, and the crossing (n - 1 with s_at = total when
-// no partial sum reaches u, as sample_from_probs falls back to the last index).
-struct SeqSum {
-    float total;
-    int cross;      // first k with u <= s_k (n-1 if none); -1 when u < 0
-    float s_at;     // s_cross
-    float s_before; // s_{cross-1} (0 for cross == 0)
-};
-
-__device__ inline SeqSum seq_sum_wave(const float* v, int n, float u) {
-    SeqScan st = seq_scan_init();
-    seq_scan_wave(v, n, u, 0, st);
-    SeqSum res;
-    res.total = st.s;
-    res.cross = st.cross;
-    res.s_at = st.s_at;
-    res.s_before = st.s_before;
-    if (u >= 0.0f && st.cross < 0) {
-        res.cross = n - 1;
-        res.s_at = st.s;
-        res.s_before = st.s;
+// Continues st over v[0..n) in LDS; lane l of isum / wexp: the integer sum of window l in ulps
+// (-1: unusable) and the binade it holds for, predicted by the caller.
+__device__ __noinline__ static SeqScan seq_scan_chunk(lds_cfloat* v, int n, float u, int gbase, SeqScan st, int isum, int wexp) {
+    n = __builtin_amdgcn_readfirstlane(n);
+    gbase = __builtin_amdgcn_readfirstlane(gbase);
+#pragma unroll 1
+    for (int w = 0; w * SCAN_WIN < n; w++) {
+        const int add = w < 64 ? __builtin_amdgcn_readlane(isum, w) : -1;
+        const int eb = w < 64 ? __builtin_amdgcn_readlane(wexp, w) : 0;
+        const uint32_t bits = (uint32_t)__builtin_amdgcn_readfirstlane(__float_as_int(st.s));
+        if (add >= 0 && (int)(bits >> 23) == eb) {
+            const int end = (int)((bits & 0x7FFFFFu) | 0x800000u) + add;
+            const float s1 = (float)end * scan_pow2(eb - 150);
+            if (end < 16777216 && !(u >= 0.0f && st.cross < 0 && u <= s1)) {
+                st.s = s1;
+                continue;
+            }
+        }
+        float x[8];
+        scan_load(v + w * SCAN_WIN, min(SCAN_WIN, n - w * SCAN_WIN), x);
+        scan_window(x, min(SCAN_WIN, n - w * SCAN_WIN), u, gbase + w * SCAN_WIN, st);
     }
-    return res;
+    return st;
 }
 
 // One 1 KiB wave load straight into LDS: lane l's 16 bytes at rsrc + voff +
