@@ -100,7 +100,7 @@ __device__ __forceinline__ float filt_exp_fast(const RowFilt& f, float l, int j,
     const bool fin = fabsf(m) < INFINITY;
     const float e = expf_fast(fin ? m - f.mx : -200.0f, b);
     bad = bad | (b & keep);
-    return keep & fin ? e : 0.0f;
+    return (keep & fin) ? e : 0.0f;
 }
 __device__ __forceinline__ float filt_prob_fast(const RowFilt& f, float l, int j, bool& bad) {
     const float p0 = div_fast(filt_exp_fast(f, l, j, bad), f.iS, bad);
