@@ -617,6 +617,25 @@ static GmPlan plan_gemm(const GemvArgs& a) {
             }
         }
     }
+    if (bkey0 < 0.0 && a.M > 32) {
+        // Nothing fits one round (long prompts).  A wave's LDS reads per k-step are 4 KiB of
+        // activations whatever its width, so a block costs about 2 + tpw tile steps and wide
+        // blocks win; ties go to the wider one.  Forwards of three layers with one tile per
+        // wave (what the search above leaves) and with this choice: INT8 d2048, 500 rows
+        // 937 -> 817 us, INT8 d4096, 400 rows 2034 -> 1801, BF16 d3072, 450 rows 1596 -> 1417,
+        // INT4 d3072, 150 rows 636 -> 599.  Up to 32 rows the loads bound the kernel and the
+        // narrow blocks stay.
+        long long bcost = 0;
+        for (int tpw = max_tpw<FMT, 2>(); tpw >= 1; tpw--) {
+            const int cap = plan_capacity<FMT, EPI>(2, 2, tpw);
+            const long long units = (long long)((ntiles + 4 * tpw - 1) / (4 * tpw)) * ((chunks + 3) / 4);
+            const long long cost = (units + cap - 1) / cap * (cap / cu_count()) * (2 + tpw);
+            if (!bcost || cost < bcost) {
+                bcost = cost;
+                best = {2, 2, tpw, 1};
+            }
+        }
+    }
     return best;
 }
 
