@@ -470,11 +470,16 @@ static double wide_time(const GemvArgs& a, int cn, int cus) {
 // from 72 to 500 rows.  The wide tiles win where their blocks fill the rounds: gate/up from 65
 // rows, qkv at 256 and 500, wo and down at 500 rows; wo and down at 256 rows (128 blocks)
 // measured 34 and 76 us against 27 and 57.  BF16 blocks cover 128 rows against 64: they
-// win where that halves the row blocks and still fills the part (183 rows: 174 us against 141).
+// win where that halves the row blocks (183 rows, which it does not: 174 us against 141) and
+// fills the dispatch rounds to nine tenths, or to three quarters where one row block reads the
+// weights from HBM once.  50304 x 3072, 200 rows (786 blocks, four rounds for three): forward
+// 888 us wide, 853 narrow; 50304 x 4096, 70 rows (393 blocks): 755 wide, 794 narrow.
 bool gemm_wide_wins(const GemvArgs& a, int cus) {
     if (a.M <= 64) return false;
-    if (a.fmt == WF_BF16)
-        return a.epi == EPI_STORE && ((a.M + 63) / 64) % 2 == 0 && blocks(a, 128, 128) * 10 >= cus * 9;
+    if (a.fmt == WF_BF16) {
+        const int nb = blocks(a, 128, 128), slots = (nb + cus - 1) / cus * cus;
+        return a.epi == EPI_STORE && ((a.M + 63) / 64) % 2 == 0 && nb * 20 >= slots * (a.M <= 128 ? 15 : 18);
+    }
     if (a.fmt != WF_INT4) return false;
     const double narrow = 5.0 + 1.75e-7 * ((a.M + 31) / 32) * (double)a.N * a.K;
     return std::min(wide_time(a, 2, cus), wide_time(a, 3, cus)) < narrow;
