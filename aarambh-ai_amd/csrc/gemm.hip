@@ -556,6 +556,12 @@ static constexpr GmTuned GM_TUNED[] = {
     {WF_BF16, 32000, 4096, {{2, 1, 2, 1}, {2, 2, 2, 1}, {2, 2, 2, 1}}},
 };
 
+bool gemm_tuned(const GemvArgs& a) {
+    for (const GmTuned& t : GM_TUNED)
+        if (t.fmt == a.fmt && t.N == a.N && t.K == a.K) return true;
+    return false;
+}
+
 // Widest weight-tile count per wave whose stage ring fits the LDS budget.
 template <int FMT, int WM>
 static constexpr int max_tpw() {

@@ -467,7 +467,9 @@ static double wide_time(const GemvArgs& a, int cn, int cus) {
 
 // gemm.hip's plans take about 5 us plus 1.75e-7 us per 32 rows, weight row and column (0.5 us
 // per 32 rows x 2048 columns x 1408 weight rows), measured within 20% for the d4096 projections
-// from 72 to 500 rows.  The wide tiles win where their blocks fill the rounds: gate/up from 65
+// from 72 to 500 rows; shapes outside its table also have blocks of 64 rows x 192 or 256
+// columns (12.5 us, then 1.33 or 1.7 us per group; gate/up 16384 x 3072 at 250 rows 57 us
+// against 65 wide, at 500 rows 108 against 122, at 333 rows 102 against 95).  The wide tiles win where their blocks fill the rounds: gate/up from 65
 // rows, qkv at 256 and 500, wo and down at 500 rows; wo and down at 256 rows (128 blocks)
 // measured 34 and 76 us against 27 and 57.  BF16 blocks cover 128 rows against 64: they
 // win where that halves the row blocks (183 rows, which it does not: 174 us against 141) and
@@ -481,7 +483,12 @@ bool gemm_wide_wins(const GemvArgs& a, int cus) {
         return a.epi == EPI_STORE && ((a.M + 63) / 64) % 2 == 0 && nb * 20 >= slots * (a.M <= 128 ? 15 : 18);
     }
     if (a.fmt != WF_INT4) return false;
-    const double narrow = 5.0 + 1.75e-7 * ((a.M + 31) / 32) * (double)a.N * a.K;
+    double narrow = 5.0 + 1.75e-7 * ((a.M + 31) / 32) * (double)a.N * a.K;
+    if (!gemm_tuned(a))  // 64-row blocks of 192 and 256 columns
+        for (int tpw = 3; tpw <= 4; tpw++) {
+            const int rounds = (blocks(a, 64 * tpw, 64) + cus - 1) / cus;
+            narrow = std::min(narrow, rounds * (12.5 + (a.K >> 7) * (tpw == 4 ? 1.7 : 1.33)));
+        }
     return std::min(wide_time(a, 2, cus), wide_time(a, 3, cus)) < narrow;
 }
 

@@ -234,6 +234,7 @@ int launch_zero_u32(uint32_t* p, int n, hipStream_t stream);
 int launch_gemv(const GemvArgs& a, hipStream_t stream);
 // Many-row variant (M > 16, fragments with mp = 16, all rows in one launch).
 int launch_gemm(const GemvArgs& a, hipStream_t stream);
+bool gemm_tuned(const GemvArgs& a);  // the shape has a measured plan
 // The same product with wide wave tiles; gemm_wide_wins: the shapes it is the faster one for.
 bool gemm_wide_wins(const GemvArgs& a, int cus);
 int launch_gemm_wide(const GemvArgs& a, int cus, hipStream_t stream);
