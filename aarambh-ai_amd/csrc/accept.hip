@@ -70,7 +70,7 @@ struct RowFilt {
     uint64_t kkey;  // top-k: logits with logit_key >= kkey are kept (0: all)
     uint64_t pkey;  // top-p: probabilities with prob_key >= pkey are kept (0: all)
     int topp;       // top-p applies
-    double iT, iS, iR2;  // reciprocals of T, S and R2 (div_fast)
+    double iT, iS, iR2;  // reciprocals of T, S and R2
 };
 
 // exp(l / T - mx) of element j (0 when top-k drops it or l / T is not finite):
@@ -96,18 +96,15 @@ __device__ __forceinline__ float filt_prob(const RowFilt& f, float l, int j) {
 __device__ __forceinline__ float filt_exp_fast(const RowFilt& f, float l, int j, bool& bad) {
     const bool keep = logit_key(l, j) >= f.kkey;
     bool b = false;
-    const float m = div_fast(l, f.iT, b);
-    const bool fin = fabsf(m) < INFINITY;
-    const float e = expf_fast(fin ? m - f.mx : -200.0f, b);
+    const float e = expf_fast(div_fast(l, f.iT) - f.mx, b);  // l / T = -inf or NaN: 0, inf: bad
     bad = bad | (b & keep);
-    return (keep & fin) ? e : 0.0f;
+    return keep ? e : 0.0f;
 }
 __device__ __forceinline__ float filt_prob_fast(const RowFilt& f, float l, int j, bool& bad) {
-    const float p0 = div_fast(filt_exp_fast(f, l, j, bad), f.iS, bad);
+    const float p0 = div_fast(filt_exp_fast(f, l, j, bad), f.iS);
     if (!f.topp) return p0;
     const bool keep = p0 > 0.0f && prob_key(p0, j) >= f.pkey;
-    const float p = div_fast(keep ? p0 : 0.0f, f.iR2, bad);
-    return p;
+    return div_fast(keep ? p0 : 0.0f, f.iR2);
 }
 
 // Row statistics handed from stage 1 to the resolving workgroup (ACC_RS_WORDS words per row).
@@ -1048,7 +1045,7 @@ __device__ __forceinline__ void row_filter(const float* row, int V, float T, int
     const SeqScan s2 = block_seq_scan<1>(
         row, nullptr, V, -1.0f,
         [&](float a, float, int j, bool& bad) {
-            const float p0 = div_fast(filt_exp_fast(fr, a, j, bad), fr.iS, bad);
+            const float p0 = div_fast(filt_exp_fast(fr, a, j, bad), fr.iS);
             return (p0 > 0.0f && prob_key(p0, j) >= fr.pkey) ? p0 : 0.0f;
         },
         [&](float a, float, int j) {
@@ -1310,7 +1307,7 @@ __global__ void __launch_bounds__(ACC_THREADS) __attribute__((amdgpu_waves_per_e
                 const double iR = 1.0 / (double)R;
                 cdf = block_seq_scan<2>(
                     tl, dl, V, u,
-                    [&](float lt, float ld, int j, bool& bad) { return div_fast(resid_fast(lt, ld, j, bad), iR, bad); },
+                    [&](float lt, float ld, int j, bool& bad) { return div_fast(resid_fast(lt, ld, j, bad), iR); },
                     [&](float lt, float ld, int j) { return resid(lt, ld, j) / R; }, lds, chunk, &sh);
             }
         } else {

@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "exact_f32.hpp"
+
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef short bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
@@ -37,45 +39,6 @@ __device__ __forceinline__ int32_t total_key(float f) {
 // correctly rounded libm expf except in the rare cases where the host libm
 // itself misrounds; those show up as flagged near-ties, never silently.
 __device__ __forceinline__ float expf_rn(float x) { return (float)exp((double)x); }
-
-// The same value without branches, or `bad` set (then expf_rn decides).  For |x| < 87 (a
-// normal f32 result) a Taylor polynomial of degree 11 on |r| <= ln 2 / 2, r = x - k ln 2,
-// gives e^x within 2^-45 relative: r^12 / 12! is below 2^-47 and the f64 roundings add a few
-// 2^-52.  Rounding it to f32 equals rounding any value within that distance, unless it lies
-// next to a midpoint of two f32 values: within 2^-42 of one (one value in 2^18) it is bad.
-// Below -104 the result is 0 (e^-104 < 2^-150).  All 2^32 inputs compared with expf_rn.
-__device__ __forceinline__ float expf_fast(float x, bool& bad) {
-    const double xd = (double)x;
-    const double k = __builtin_rint(xd * 1.4426950408889634);
-    const double r = fma(-k, 0.6931471805599453, xd);
-    double p = 1.0 / 39916800.0;
-    p = fma(p, r, 1.0 / 3628800.0);
-    p = fma(p, r, 1.0 / 362880.0);
-    p = fma(p, r, 1.0 / 40320.0);
-    p = fma(p, r, 1.0 / 5040.0);
-    p = fma(p, r, 1.0 / 720.0);
-    p = fma(p, r, 1.0 / 120.0);
-    p = fma(p, r, 1.0 / 24.0);
-    p = fma(p, r, 1.0 / 6.0);
-    p = fma(p, r, 0.5);
-    p = fma(p, r, 1.0);
-    p = fma(p, r, 1.0);
-    // the 29 bits below f32 precision, measured from the midpoint (2^28) in units of 2^-52
-    const uint32_t d = ((uint32_t)__double2loint(p) & 0x1FFFFFFFu) - (0x10000000u - 1024u);
-    const bool zero = x < -104.0f;
-    bad = bad | ((!(fabsf(x) < 87.0f) | (d <= 2048u)) & !zero);
-    return zero ? 0.0f : (float)__builtin_ldexp(p, (int)k);
-}
-
-// x / d, correctly rounded, with inv = 1 / (double)d and no branch.  The quotient of two 24-bit
-// numbers lies at least 2^-49 (relative) from every midpoint of two f32 values, and x * inv
-// in f64 within 2^-51.9 of it, so both round to the same f32.  `bad` is set for results near
-// the subnormal range (where f32 has fewer bits) and NaN: then x / d decides.
-__device__ __forceinline__ float div_fast(float x, double inv, bool& bad) {
-    const float y = (float)((double)x * inv);
-    bad = bad | !((fabsf(y) > 1e-30f) | (x == 0.0f));
-    return y;
-}
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 __device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
