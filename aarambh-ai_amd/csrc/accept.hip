@@ -24,6 +24,7 @@
 
 #include "device_common.hpp"
 #include "kernels.hpp"
+#include "row_slot.hpp"
 
 namespace aarh {
 
@@ -1120,8 +1121,8 @@ __global__ void __launch_bounds__(ACC_THREADS) __attribute__((amdgpu_waves_per_e
     const int lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int rows_per_seq = a.target_rows + a.K;
-    const int b = blockIdx.x / rows_per_seq;
-    const int r = blockIdx.x % rows_per_seq;
+    const RowSlot slot = row_slot((int)blockIdx.x, (int)gridDim.x, rows_per_seq, a.cus);
+    const int b = __builtin_amdgcn_readfirstlane(slot.seq), r = __builtin_amdgcn_readfirstlane(slot.row);
     const int V = a.V;
     const int chunk = a.chunk;
     int np = a.n_proposals ? a.n_proposals[b] : a.K;
@@ -1349,6 +1350,16 @@ static size_t accept_lds_bytes(int V, int greedy, int top_p_active, int top_k) {
     return f * sizeof(float);
 }
 
+static int accept_cus() {
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        (void)hipGetDevice(&dev);
+        (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+        return n > 0 ? n : 256;
+    }();
+    return cus;
+}
+
 int launch_accept(const AcceptArgs& a_in, hipStream_t stream) {
     AcceptArgs a = a_in;
     const int rows = a.target_rows + a.K;
@@ -1357,6 +1368,9 @@ int launch_accept(const AcceptArgs& a_in, hipStream_t stream) {
     if (lds > MAX_DYN_LDS) return 3;
     a.chunk = a.V < ACC_CHUNK ? a.V : ACC_CHUNK;
     if (a.chunk < 1) a.chunk = 1;
+    // greedy and compact top-k resolvers are short, and their rows gain nothing from pairs (top-k
+    // 50, 32 sequences x 9 rows: 135 us in row order, 139 in pairs; 64 sequences: 155 and 151)
+    a.cus = a.greedy || topk_compact(a.top_k, a.V) ? a.B * rows : accept_cus();
     static std::once_flag once;
     static hipError_t attr = hipSuccess;
     std::call_once(once, [] {

@@ -200,6 +200,7 @@ struct AcceptArgs {
     uint32_t* rstat;      // [B * (target_rows + K)][ACC_RS_WORDS] row parameters (scratch)
     unsigned* counters;   // [B] arrival counters, zero between launches
     int chunk;            // set by the launcher
+    int cus;              // compute units (row_slot), set by the launcher
     int32_t* out_accept_len;
     int32_t* out_token;
     uint32_t* out_flags;
