@@ -83,10 +83,6 @@ __device__ __forceinline__ void store_kv_token(const AttnArgs& a, size_t hb, int
         }
     }
 }
-__device__ __forceinline__ void append_kv_token(const AttnArgs& a, int seq, int kvh, size_t hb, int pos0, int t) {
-    store_kv_token(a, hb, t, load_kv_token(a, seq, kvh, pos0, t));
-}
-
 // Append this launch's new positions that fall in [t_begin, t_end), spread over the
 // workgroup's waves.  Every workgroup whose chunk covers a new position writes it
 // (identical bytes) before it reads the chunk, so no other launch is needed.
@@ -95,7 +91,14 @@ __device__ void append_new_kv(const AttnArgs& a, int seq, int kvh, size_t hb, in
     const int lo = max(t_begin, pos0);
     if (lo >= t_end) return;  // uniform over the workgroup
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
-    for (int t = lo + wid; t < t_end; t += nw) append_kv_token(a, seq, kvh, hb, pos0, t);
+    for (int t = lo + wid; t < t_end; t += 4 * nw) {  // four rows in one round trip
+        KvNew nv[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) nv[j] = load_kv_token(a, seq, kvh, pos0, min(t + j * nw, t_end - 1));
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (t + j * nw < t_end) store_kv_token(a, hb, t + j * nw, nv[j]);
+    }
     __threadfence_block();
     __syncthreads();
 }
@@ -332,8 +335,8 @@ static constexpr int AM_HD = 128;
 static constexpr int AM_WAVES = 8;          // 512 threads; wave w takes 32-token blocks w, w+8, ...
 static constexpr int AM_TAIL = AM_WAVES - 1;  // INT8 path: the wave that appends and reads the new positions
 static constexpr int AM_HAND = 2;             // old blocks the tail wave hands over beyond its tail blocks
-// Rows per sequence up to which the new positions (at most two blocks) are appended inside
-// the attention kernel; prompt chunks beyond it are appended by a launch of their own.
+// INT8 path: rows per sequence up to which the new positions are appended inside the attention
+// kernel (they lie in at most two blocks, which one wave can take); append_first has the rule.
 static constexpr int AM_DECODE_S = 32;
 static constexpr int AM_REC = AM_HD + 4;    // partial record: m, l, pad, pad, o[hd]
 static constexpr int AM_MAXCH = 32;         // chunks one merge combines
@@ -444,8 +447,8 @@ __device__ __forceinline__ void frag_out_pair(const XFrag& fo, int orow, int oco
     frag_put8_w(fo, orow, ocol, v);
 }
 
-// Cache append of a prompt chunk (S > AM_DECODE_S): workgroup = (sequence, kv head, 32-token
-// block of the cache).  The block's new rows are rounded as append_kv_token rounds them into
+// Cache append of a prompt chunk (append_first): workgroup = (sequence, kv head, 32-token
+// block of the cache).  The block's new rows are rounded as store_kv_token rounds them into
 // an LDS copy of the block (loaded first where the block also holds older tokens) and the
 // block goes to the cache in 16-byte runs.  One rounding per new token: appended inside the
 // attention kernel, every 16-row query tile rounded every new token again (32 / 8 heads of
@@ -524,8 +527,8 @@ __global__ void __launch_bounds__(256) kv_append_kernel(AttnArgs a, int nblk) {
 // the lane of their row.  Softmax runs in base 2 (v_exp_f32).  With one chunk
 // the workgroup writes the output; otherwise chunk partials go out with
 // coherent 16-byte stores and the last workgroup of the group merges them.
-// PRE: the new positions are in the cache already (kv_append_kernel) and each query tile
-// reads only the blocks up to its last row's position.
+// PRE: the new positions are in the cache already (kv_append_kernel).  With PRE, and in the
+// fp16 path, each query tile reads (and appends) only up to its last row's position.
 template <int KVF, int DEPTH, bool DMA, bool PRE>
 __global__ void __launch_bounds__(512) attn_mfma_kernel(AttnArgs a) {
     // dynamic LDS: the DMA block stages during the token loop, then the wave merge
@@ -553,9 +556,10 @@ __global__ void __launch_bounds__(512) attn_mfma_kernel(AttnArgs a) {
     const int QD = a.n_heads * AM_HD;
     const size_t hb = (size_t)sl * a.n_kv + kvh;
     const int t_begin = chunk * a.chunk;
-    const int seen = PRE ? pos0 + (r0 + R - 1) / G + 1 : kv_len;  // tokens the tile's rows attend to
+    constexpr bool STOP = PRE || !DMA;
+    const int seen = STOP ? pos0 + (r0 + R - 1) / G + 1 : kv_len;  // tokens the tile's rows attend to
     const int t_end = min(seen, t_begin + a.chunk);
-    const int lim0 = PRE ? pos0 + r0 / G : pos0;  // tokens up to here are seen by every row
+    const int lim0 = STOP ? pos0 + r0 / G : pos0;  // tokens up to here are seen by every row
     constexpr int STEP = 32 * AM_WAVES;
     int tb = t_begin + 32 * wid;
     const int t_chunk_last = (t_end - 1) & ~31;
@@ -606,7 +610,7 @@ __global__ void __launch_bounds__(512) attn_mfma_kernel(AttnArgs a) {
         return t_begin + 32 * (AM_TAIL + AM_WAVES * (t_old - n_moved + i - n_first));  // handed over
     };
     // The cache append of tail block tb (positions max(tb, pos0) .. min(tb + 32, t_end) - 1,
-    // the bytes append_kv_token writes), made in the block's landed stage; the patched
+    // the bytes store_kv_token writes), made in the block's landed stage; the patched
     // block then goes back to the cache whole, in the 16-byte runs the loads read.
     // The wave holding the first tail block loads the first four new rows before any
     // block (ahead of the block loads in the memory pipeline); other rows are loaded
@@ -924,13 +928,26 @@ static int launch_mfma_pre(const AttnArgs& a, int grid, hipStream_t stream) {
     return note_error(hipGetLastError()) ? 4 : 0;
 }
 
-// Up to AM_DECODE_S rows per sequence (verify, replay, decode) the new positions lie in at
-// most two blocks and the kernel appends them itself: the append launch would cost such a
-// forward 8-10 us per layer where its attention takes 15-20.  Prompt chunks append first
-// and skip the blocks their rows do not see.
+// Whether the new positions are appended by a launch of their own before the attention.
+// INT8: beyond AM_DECODE_S rows per sequence.  Up to there the append launch would cost a
+// forward 8-10 us per layer where its attention takes 15-20; beyond, the in-kernel append holds
+// every query tile up more than that (d_model 4096, 33 rows over 3000 tokens, two layers: 437 us
+// in the kernel, 336 with the launch; 64 rows 379 and 343).
+// fp16: every query tile rounds the new rows up to its own, without a reduction, so the launch
+// pays only for more of them: beyond 96 rows, or where the tiles of all sequences round more than
+// 14000 rows (rows x tiles; never for decode and verify).  Two layers, d_model 2048 (4 kv heads of 4 query heads), over 1000
+// tokens: 33 rows 212 us in the kernel, 231 with the launch, 64 rows 219 and 236, 96 rows 263
+// and 270, 128 rows 274 and 268; d_model 4096 (8 kv heads of 4): 64 rows 312 and 322, 80 rows
+// 391 and 393, 96 rows (18 432) 406 and 396; four sequences of d_model 2048 over 2000 tokens:
+// 48 rows 338 and 340, 64 rows (16 384) 367 and 356.
+static bool append_first(const AttnArgs& a) {
+    if (a.kv_fmt == KV_INT8) return a.S > AM_DECODE_S;
+    return a.S > 96 || (a.S > 32 && (long long)a.S * a.nseq * a.n_kv * a.ntiles > 14000);
+}
+
 template <int KVF, bool DMA>
 static int launch_mfma(const AttnArgs& a, int grid, hipStream_t stream) {
-    if (a.S <= AM_DECODE_S) return launch_mfma_pre<KVF, DMA, false>(a, grid, stream);
+    if (!append_first(a)) return launch_mfma_pre<KVF, DMA, false>(a, grid, stream);
     const int nblk = (a.S + 30) / 32 + 1;  // cache blocks that S positions can touch
     launch_timed(kv_append_kernel<KVF>, dim3(a.nseq * a.n_kv * nblk), dim3(256), 0, stream, a, nblk);
     return launch_mfma_pre<KVF, DMA, true>(a, grid, stream);
