@@ -91,14 +91,7 @@ __device__ void append_new_kv(const AttnArgs& a, int seq, int kvh, size_t hb, in
     const int lo = max(t_begin, pos0);
     if (lo >= t_end) return;  // uniform over the workgroup
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
-    for (int t = lo + wid; t < t_end; t += 4 * nw) {  // four rows in one round trip
-        KvNew nv[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) nv[j] = load_kv_token(a, seq, kvh, pos0, min(t + j * nw, t_end - 1));
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            if (t + j * nw < t_end) store_kv_token(a, hb, t + j * nw, nv[j]);
-    }
+    for (int t = lo + wid; t < t_end; t += nw) store_kv_token(a, hb, t, load_kv_token(a, seq, kvh, pos0, t));
     __threadfence_block();
     __syncthreads();
 }
@@ -556,10 +549,10 @@ __global__ void __launch_bounds__(512) attn_mfma_kernel(AttnArgs a) {
     const int QD = a.n_heads * AM_HD;
     const size_t hb = (size_t)sl * a.n_kv + kvh;
     const int t_begin = chunk * a.chunk;
-    constexpr bool STOP = PRE || !DMA;
-    const int seen = STOP ? pos0 + (r0 + R - 1) / G + 1 : kv_len;  // tokens the tile's rows attend to
+    const bool stop = PRE || (!DMA && a.ntiles > 1);
+    const int seen = stop ? pos0 + (r0 + R - 1) / G + 1 : kv_len;  // tokens the tile's rows attend to
     const int t_end = min(seen, t_begin + a.chunk);
-    const int lim0 = STOP ? pos0 + r0 / G : pos0;  // tokens up to here are seen by every row
+    const int lim0 = stop ? pos0 + r0 / G : pos0;  // tokens up to here are seen by every row
     constexpr int STEP = 32 * AM_WAVES;
     int tb = t_begin + 32 * wid;
     const int t_chunk_last = (t_end - 1) & ~31;
@@ -935,11 +928,13 @@ static int launch_mfma_pre(const AttnArgs& a, int grid, hipStream_t stream) {
 // in the kernel, 336 with the launch; 64 rows 379 and 343).
 // fp16: every query tile rounds the new rows up to its own, without a reduction, so the launch
 // pays only for more of them: beyond 96 rows, or where the tiles of all sequences round more than
-// 14000 rows (rows x tiles; never for decode and verify).  Two layers, d_model 2048 (4 kv heads of 4 query heads), over 1000
-// tokens: 33 rows 212 us in the kernel, 231 with the launch, 64 rows 219 and 236, 96 rows 263
-// and 270, 128 rows 274 and 268; d_model 4096 (8 kv heads of 4): 64 rows 312 and 322, 80 rows
-// 391 and 393, 96 rows (18 432) 406 and 396; four sequences of d_model 2048 over 2000 tokens:
-// 48 rows 338 and 340, 64 rows (16 384) 367 and 356.
+// 14000 rows (rows x tiles; never for decode and verify).  Two layers, d_model 2048 (4 kv heads
+// of 4 query heads), over 1000 tokens: 33 rows 213 us in the kernel, 232 with the launch, 64 rows
+// 218 and 238, 96 rows 266 and 272, 128 rows 275 and 268; d_model 4096 (8 kv heads of 4): 64 rows
+// 306 and 319, 80 rows (12 800) 385 and 394, 96 rows (18 432) 412 and 393; four sequences of
+// d_model 2048: 48 rows over 100 tokens 291 and 302, over 2000 344 and 340, 64 rows (16 384) over
+// 2000 372 and 352.  (Four new rows per round trip took 2% off such chunks and cost verify
+// attention 0.5-0.9 us of 19.)
 static bool append_first(const AttnArgs& a) {
     if (a.kv_fmt == KV_INT8) return a.S > AM_DECODE_S;
     return a.S > 96 || (a.S > 32 && (long long)a.S * a.nseq * a.n_kv * a.ntiles > 14000);

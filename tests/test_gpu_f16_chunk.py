@@ -57,7 +57,7 @@ def attention_us(m, rows, ctx):
 
 
 def test_f16_short_chunk_time():
-    """33 rows pay for one more query tile, not for an append launch (19 against 29 us)."""
+    """33 rows pay for one more query tile, not for an append launch (15 us against 24)."""
     m = A.HipModel(A.ModelConfig(vocab_size=512, hidden_dim=2048, ffn_dim=512, n_layers=4, n_heads=16, n_kv_heads=4,
                                  max_seq_len=1100, weight_format=A.W_INT8_ROW, kv_format=A.KV_F16, lm_head_format=1),
                    max_batch=1, max_rows=64)
