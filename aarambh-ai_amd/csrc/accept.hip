@@ -340,7 +340,7 @@ __device__ __forceinline__ uint64_t select_desc(const KF& kf, const float* row, 
 // other waves write chunk c + 1 into the other half.
 //
 // Before the scan of a chunk all waves sum its windows of SCAN_WIN values: inside one binade
-// the running sum grows by the integer sum of RNE(x / ulp) (see seq_scan_wave), which does
+// the running sum grows by the integer sum of RNE(x / ulp) (see scan_window), which does
 // not depend on the sum itself, only on its binade.  The binade at each window's start is
 // predicted from plain f32 sums; the scan uses a window's integer sum only where the
 // running sum is in that binade and stays in it, no element is special and the draw u is not
@@ -348,9 +348,10 @@ __device__ __forceinline__ uint64_t select_desc(const KF& kf, const float* row, 
 // for each doubling of the sum).  So the prediction decides the time and never the result.
 // What bounds it now is the producing: with two exact exponentials and five exact quotients per
 // residual, one workgroup writes an 8192-value chunk in 6-12 us, against 3-5 us for scanning
-// it (10-15 us for the first chunk, whose sum doubles every few values).  32 sequences x 9
-// rows of 32 000 logits at temperature 0.8: 254 us before the window sums, the branch-free
-// producers and the parallel acceptance probabilities, 232 us with them.
+// it (10-15 us for the first chunk, whose sum doubles every few values).  28 sequences x 9
+// rows of 32 000 logits at temperature 0.8: 208 us before the window sums, the branch-free
+// producers and the parallel acceptance probabilities, 180 us with them (32 sequences, whose
+// workgroups share compute units: 226 and, with row_slot, 186).
 static_assert(ACC_CHUNK <= 2 * ACC_WAVES * SCAN_WIN, "two windows per wave");
 typedef __attribute__((address_space(3))) ScanShared lds_scan;
 __device__ __noinline__ static void scan_windows(lds_cfloat* buf, int m, float s0, lds_scan* sh) {
@@ -594,7 +595,7 @@ __device__ __forceinline__ float surv_logit(unsigned long long k) { return __uin
 
 // Inverse CDF of sample_from_probs (sampler.rs:337-347) over survivors in index order
 // with values v[i] / div (div = 1: the values themselves), on thread 0: the first index
-// with u <= cumulative, as seq_scan_wave reports it (u <= 0 stops at index 0 with the
+// with u <= cumulative, as seq_scan_chunk reports it (u <= 0 stops at index 0 with the
 // partial sums 0).
 __device__ inline SeqScan block_cdf_small(const unsigned long long* keys, const float* v, int n, float div, float u,
                                           AccShared* sh) {

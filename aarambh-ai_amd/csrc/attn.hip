@@ -465,7 +465,7 @@ __global__ void __launch_bounds__(256) kv_append_kernel(AttnArgs a, int nblk) {
     const int lo = max(tb, pos0), hi = min(tb + 32, kv_len);
     char* kb = (char*)a.kc + (hb * a.cap + tb) * AM_HD * ES;
     char* vb = (char*)a.vc + (hb * a.cap + tb) * AM_HD * ES;
-    // the four rows of a wave's next step in one round trip
+    // the wave's eight rows in one round trip
     KvNew nv[8];
 #pragma unroll
     for (int j = 0; j < 8; j++) nv[j] = load_kv_token(a, seq, kvh, pos0, min(max(tb + wid + 4 * j, lo), hi - 1));

@@ -22,13 +22,8 @@ __device__ __forceinline__ void gemm_tail(const GemvArgs& a, int S, int s, int m
     //      same round trip as the split-K partials (after the arrival, which waits for
     //      every outstanding access), or right away without a split ----
     int ntv[TPW];
-    bool tok[TPW];
 #pragma unroll
-    for (int j = 0; j < TPW; j++) {
-        const int nt = tile0 + j;
-        tok[j] = nt < ntiles;
-        ntv[j] = min(nt, ntiles - 1);
-    }
+    for (int j = 0; j < TPW; j++) ntv[j] = min(tile0 + j, ntiles - 1);
     // RESID: unit u = (row r, 8-column half s8 of a tile) of the wave's region; the old
     // residual and the next consumer's norm weights of every unit of the lane
     constexpr int TR = 16 * CPW, TLD = 16 * TPW + 4;
