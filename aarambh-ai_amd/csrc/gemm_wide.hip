@@ -22,9 +22,8 @@
 // INT4 d4096 layers: gate/up at 128 rows 55.5 -> 49.5 us; at 500 rows qkv 66 -> 59, wo 50 ->
 // 40, gate/up 208 -> 200, down 110 -> 90 us.  LM head 32000 x 4096: 72 rows 112 -> 86, 128
 // rows 98.6 -> 94.5, 500 rows 357 -> 329 us.
-#include <algorithm>
-
 #include "gemm_tail.hpp"
+#include "gemm_wide_rule.hpp"
 
 namespace aarh {
 
@@ -72,10 +71,10 @@ struct GwCfg {
     static constexpr int STAGE = WK * AB + WN * WB;
     static constexpr int ZW = I4 ? 256 * ((CN + 3) / 4) : 0;
     static constexpr int WZ = I4 ? NWV * (CN * 1024 + ZW) : 0;  // INT4 weight + scale slot
-    // stages: three where they fit, else two (INT4 keeps one weight slot less than stages)
-    static constexpr int NS = 3 * STAGE + 2 * WZ <= GW_LDS ? 3 : 2;
-    static constexpr int NW = I4 ? NS - 1 : 0;
-    static constexpr int LDS = NS * STAGE + NW * WZ;
+    // stages: three where they fit, else two (INT4: two, and one weight slot)
+    static constexpr int NS = 3 * STAGE + WZ <= GW_LDS ? 3 : 2;
+    static_assert(!I4 || NS == 2, "the INT4 loop refills its one weight slot once a stage");
+    static constexpr int LDS = NS * STAGE + WZ;
     static constexpr int LA = CM * SG * 2 / WN;             // activation loads per wave and stage
     static constexpr int LW = I4 ? CN + (CN + 3) / 4 : CN * SG / WM;  // weight (and scale) loads
     static constexpr int CPW = CM / WK;                     // chunks a wave keeps after the K reduction
@@ -143,17 +142,17 @@ __global__ void __launch_bounds__(WM * WN * WK * 64, 1) gemm_wide_kernel(GemvArg
             }
         }
     };
-    auto issue_w = [&](int i, int slot) {
+    auto issue_w = [&](int i) {
         if constexpr (C::I4) {
             const int g = grp(i);
 #pragma unroll
             for (int j = 0; j < CN; j++)
-                lds_dma16<true>(wr, w_lds + slot * C::WZ + j * 1024, lane * 16,
+                lds_dma16<true>(wr, w_lds + j * 1024, lane * 16,
                              (int)(((unsigned)min(nt0 + j, ntiles - 1) * G + g) * 1024u));
 #pragma unroll
             for (int q = 0; q < (CN + 3) / 4; q++) {
                 const int zt = min(nt0 + min(4 * q + (lane >> 4), CN - 1), ntiles - 1);
-                lds_dma4(zr, w_lds + slot * C::WZ + CN * 1024 + q * 256, (int)(((unsigned)zt * G + g) * 64u + lr * 4u), 0);
+                lds_dma4(zr, w_lds + CN * 1024 + q * 256, (int)(((unsigned)zt * G + g) * 64u + lr * 4u), 0);
             }
         }
     };
@@ -183,12 +182,9 @@ __global__ void __launch_bounds__(WM * WN * WK * 64, 1) gemm_wide_kernel(GemvArg
             for (int u = 0; u < 4; u++) iv[k][u] = a.ssq_in[(size_t)m * a.ssq_ld + min(lane + 64 * u, nq - 1)];
         }
     }
-    issue_w(0, 0);
+    issue_w(0);
     issue_stage(0, 0);
-    if constexpr (NS == 3) {
-        issue_w(1, C::NW > 1 ? 1 : 0);
-        issue_stage(1, 1);
-    }
+    if constexpr (NS == 3) issue_stage(1, 1);
     issue_stage(NS - 1, NS - 1);
     if (norm_rows && !inv_late) {
         float ss[RPW];
@@ -256,12 +252,11 @@ __global__ void __launch_bounds__(WM * WN * WK * 64, 1) gemm_wide_kernel(GemvArg
             for (int j = 0; j < CN; j++)
                 wb[buf][j] = ((const u32x4_t*)(w_ptr + slot * C::STAGE + (j * C::SG + tt) * 1024))[lane];
     };
-    auto read_w = [&](int slot, u32x4_t (&w)[CN], uint32_t (&z)[CN]) {
-        const char* base = w_ptr + slot * C::WZ;
+    auto read_w = [&](u32x4_t (&w)[CN], uint32_t (&z)[CN]) {
 #pragma unroll
         for (int j = 0; j < CN; j++) {
-            w[j] = ((const u32x4_t*)(base + j * 1024))[lane];
-            z[j] = ((const uint32_t*)(base + CN * 1024 + j * 64))[lr];
+            w[j] = ((const u32x4_t*)(w_ptr + j * 1024))[lane];
+            z[j] = ((const uint32_t*)(w_ptr + CN * 1024 + j * 64))[lr];
         }
     };
     half2_t zl2[CN], zh2[CN];
@@ -313,14 +308,13 @@ __global__ void __launch_bounds__(WM * WN * WK * 64, 1) gemm_wide_kernel(GemvArg
     __syncthreads();
     read_a(0, 0, 0);
     if constexpr (C::I4) {
-        read_w(0, wb[0], szw);
+        read_w(wb[0], szw);
         prep_z();
         wait_lds();
-        issue_w(C::NW, 0);
+        issue_w(1);
     }
     int sl = 0;
     if constexpr (C::I4) {
-        int ws = 0;  // weight slot of the group in registers
         for (int i = 0; i < n_it; i++) {
             u32x4_t wn_[CN];
             uint32_t zn_[CN];
@@ -339,10 +333,9 @@ __global__ void __launch_bounds__(WM * WN * WK * 64, 1) gemm_wide_kernel(GemvArg
             boundary();
             issue_stage(i + NS, sl);
             sl = next(sl);
-            ws = ws + 1 == C::NW ? 0 : ws + 1;
             SCHED_FENCE;
             read_a(0, sl, 0);
-            read_w(ws, wn_, zn_);
+            read_w(wn_, zn_);
             SCHED_FENCE;
             mfma_t(1, 3);
             const bool on = i < my_n;
@@ -360,7 +353,7 @@ __global__ void __launch_bounds__(WM * WN * WK * 64, 1) gemm_wide_kernel(GemvArg
             }
             prep_z();
             wait_lds();  // the slot's words have been read
-            issue_w(i + 1 + C::NW, ws);
+            issue_w(i + 2);
         }
     } else {
         for (int h = 0; h < 2 * n_it; h++) {
@@ -453,43 +446,9 @@ static int launch_wide_cfg(const GemvArgs& a, hipStream_t stream) {
     return note_error(hipGetLastError()) ? 4 : 0;
 }
 
-static int blocks(const GemvArgs& a, int cols, int rows) {
-    return ((a.N + cols - 1) / cols) * ((a.M + rows - 1) / rows);
-}
-
-// INT4: tile width (2 or 3 weight tiles per wave: 128 or 192 columns x 64 rows per block) and
-// time in us of a launch without k-splits, from the measured cost of a block (10 us of ramp, K
-// reduction and epilogue, then 0.93 or 1.22 us per 128-column group) and the dispatch rounds.
-static double wide_time(const GemvArgs& a, int cn, int cus) {
-    const int rounds = (blocks(a, 64 * cn, 64) + cus - 1) / cus;
-    return rounds * (10.0 + (a.K >> 7) * (cn == 3 ? 1.22 : 0.93));
-}
-
-// gemm.hip's plans take about 5 us plus 1.75e-7 us per 32 rows, weight row and column (0.5 us
-// per 32 rows x 2048 columns x 1408 weight rows), measured within 20% for the d4096 projections
-// from 72 to 500 rows; shapes outside its table also have blocks of 64 rows x 192 or 256
-// columns (12.5 us, then 1.33 or 1.7 us per group; gate/up 16384 x 3072 at 250 rows 57 us
-// against 65 wide, at 500 rows 108 against 122, at 333 rows 102 against 95).  The wide tiles win where their blocks fill the rounds: gate/up from 65
-// rows, qkv at 256 and 500, wo and down at 500 rows; wo and down at 256 rows (128 blocks)
-// measured 34 and 76 us against 27 and 57.  BF16 blocks cover 128 rows against 64: they
-// win where that halves the row blocks (183 rows, which it does not: 174 us against 141) and
-// fills the dispatch rounds to nine tenths, or to three quarters where one row block reads the
-// weights from HBM once.  50304 x 3072, 200 rows (786 blocks, four rounds for three): forward
-// 888 us wide, 853 narrow; 50304 x 4096, 70 rows (393 blocks): 755 wide, 794 narrow.
 bool gemm_wide_wins(const GemvArgs& a, int cus) {
-    if (a.M <= 64) return false;
-    if (a.fmt == WF_BF16) {
-        const int nb = blocks(a, 128, 128), slots = (nb + cus - 1) / cus * cus;
-        return a.epi == EPI_STORE && ((a.M + 63) / 64) % 2 == 0 && nb * 20 >= slots * (a.M <= 128 ? 15 : 18);
-    }
-    if (a.fmt != WF_INT4) return false;
-    double narrow = 5.0 + 1.75e-7 * ((a.M + 31) / 32) * (double)a.N * a.K;
-    if (!gemm_tuned(a))  // 64-row blocks of 192 and 256 columns
-        for (int tpw = 3; tpw <= 4; tpw++) {
-            const int rounds = (blocks(a, 64 * tpw, 64) + cus - 1) / cus;
-            narrow = std::min(narrow, rounds * (12.5 + (a.K >> 7) * (tpw == 4 ? 1.7 : 1.33)));
-        }
-    return std::min(wide_time(a, 2, cus), wide_time(a, 3, cus)) < narrow;
+    if (a.fmt == WF_BF16) return a.epi == EPI_STORE && wide_wins_head(a.N, a.M, cus);
+    return a.fmt == WF_INT4 && wide_wins_int4(a.N, a.K, a.M, gemm_tuned(a), cus);
 }
 
 template <int EPI>
@@ -498,7 +457,8 @@ static int launch_wide_epi(const GemvArgs& a, int cus, hipStream_t stream) {
         if constexpr (EPI == EPI_STORE) return launch_wide_cfg<WF_BF16, EPI, 4, 2, 2, 4, 1>(a, stream);
         return 2;
     }
-    if (wide_time(a, 3, cus) <= wide_time(a, 2, cus)) return launch_wide_cfg<WF_INT4, EPI, 4, 3, 1, 4, 2>(a, stream);
+    if (wide_time(a.N, a.K, a.M, 3, cus) <= wide_time(a.N, a.K, a.M, 2, cus))
+        return launch_wide_cfg<WF_INT4, EPI, 4, 3, 1, 4, 2>(a, stream);
     return launch_wide_cfg<WF_INT4, EPI, 4, 2, 1, 4, 2>(a, stream);
 }
 
