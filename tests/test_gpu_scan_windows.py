@@ -34,14 +34,17 @@ def test_window_edges_match_sequential_sums(V):
                                  max_seq_len=16), max_batch=1, max_rows=16)
     dev = torch.device("cuda:0")
     K, T = 2, 0.9
+    first = last = 0
     for i, kind in enumerate(["normal", "equal", "wide", "masked", "peak"]):
         rng = np.random.default_rng([V, i])
         B = 6
         tgt = rows(kind, rng, (B, K + 1, V))
         drf = (tgt[:, :K] + np.where(np.isfinite(tgt[:, :K]), rng.normal(0, 1, (B, K, V)), 0)).astype(np.float32)
         toks = np.where(np.isfinite(drf), drf, -1e9).argmax(-1).astype(np.uint32)
-        # uniforms near 0 and 1 put the draws into the first and the last window
-        u = np.tile(np.array([[0.999, 0.5, 0.9999], [1e-7, 0.3, 0.999999], [0.7, 0.95, 1e-7]], np.float32), (2, 1))
+        # the resampled or bonus draw lies in the first window, in the last one and between (a draw
+        # within 1e-6 of a partial sum is flagged and not compared, so none is smaller than 1e-3)
+        u = np.array([[0.999, 0.5, 0.9999], [1e-7, 0.3, 0.9997], [0.7, 0.95, 1e-3], [0.9999, 2e-3, 0.5],
+                      [0.02, 0.9998, 2e-3], [1e-7, 1e-7, 0.0015]], np.float32)
         for top_p in (0.0, 0.9):
             s = A.Sampler.top_k_top_p(T, top_p=top_p)
             t = lambda a: torch.from_numpy(a).to(dev)
@@ -56,4 +59,8 @@ def test_window_edges_match_sequential_sums(V):
             flagged = (ref["flags"] != 0) | (out["flags"] != 0)
             same = (out["accept_len"] == ref["accept_len"]) & (out["token"] == ref["token"]) & (out["draws"] == ref["draws"])
             assert (same | flagged).all(), (kind, top_p, out, ref)
+            assert (~flagged).sum() >= 3, (kind, top_p, ref)
+            first += int((~flagged & (out["token"] < 512)).sum())
+            last += int((~flagged & (out["token"] >= V - 512)).sum())
+    assert first >= 12 and last >= 6, (first, last)  # crossings in the first and the last window that were compared
     m.close()
