@@ -331,9 +331,9 @@ __device__ __forceinline__ void scan_window(const float (&x)[8], int n, float u,
         // Zero and subnormal sums count in the ulps of the first binade, 2^-149, where every
         // increment is exact.  Sums below 2^-103 are counted with all values times 2^64 (exact,
         // or infinite and so special).  At low temperatures a row's sum stays there until its
-        // first sizable term.  With the lanes of such windows added one by one, 32 sequences x 9
-        // rows of 32 000 logits took 421 us at temperature 0.1 and 2510 us at 0.02 (one lane is
-        // 0.4 us); counted this way 222 and 227 us, as at ordinary temperatures.
+        // first sizable term.  With the lanes of such windows added one by one, 28 sequences x 9
+        // rows of 32 000 logits took 419 us at temperature 0.1 and 2512 us at 0.02 (one lane is
+        // 0.4 us); counted this way 167 and 174 us, as at ordinary temperatures.
         const int eb = max((int)(bits >> 23), 1);
         const bool tiny = eb < SCAN_MIN_EB;
         const float up = tiny ? 0x1p64f : 1.0f, down = tiny ? 0x1p-64f : 1.0f;
